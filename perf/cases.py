@@ -1,0 +1,755 @@
+"""The measured cases: what a user of this package has it do, through its public entry points.
+
+Each case is one call sequence of :mod:`solprop_amd.native` or
+:mod:`solprop_amd.surrogate`: a march, a probe trial, a session, a replay, a scan, or
+the surrogate's training and screening. ``prepare`` builds what a program holds before
+the call (the problem, its workspace, the launch field in host memory), ``run`` makes the
+call and returns the fields and rows it yields, and ``exact`` is the same result from
+plain torch in 64 bits where a closed sequence of operations defines it (the adaptive
+marches have none beside another controller).
+"""
+
+from __future__ import annotations
+
+import dataclasses
+import functools
+import math
+
+import numpy as np
+import torch
+
+from solprop_amd import surrogate
+from solprop_amd.native import Scan, Workspace
+from solprop_amd.problem import (
+    capillary_problem,
+    cartesian_problem,
+    gnlse_problem,
+    radial_problem,
+)
+
+C_LIGHT = 299792458.0
+EPS0 = 8.8541878188e-12
+SCAN_DT = 400e-15 / 2**14  # every scan instance keeps the capillary grid's spacing
+
+
+# ------------------------------------------------------------------------------ cases
+
+
+def listed():
+    return [
+        # A fibre pulse propagated between two output planes: the GNLSE builder's own
+        # grid (2^13 bins, Raman, shot noise), the embedded Runge-Kutta march.
+        dict(name="fibre_march", kind="envelope_march", n_t=8192, ffac=2, soliton=4.0,
+             absorber="none", noise="input", attempts=40),
+        # One probe trial on a wide, finely sampled supercontinuum window: the largest
+        # envelope transform (2^18 samples of the Raman drive).
+        dict(name="fibre_wide_trial", kind="envelope_trial", n_t=65536, ffac=2, soliton=8.0,
+             absorber="in_stage", noise="modified", dz=2e-4),
+        # One point of a parameter scan run as a driver's session, with plane statistics
+        # every few steps: the smallest field march (one mode, 2^12 samples, 32 nodes).
+        dict(name="point_session", kind="session", n_t=4096, modes=1, nodes=32, pressure=1.2,
+             energy=120e-6, fwhm=12e-15, observations=6, every=8),
+        # The gas-filled capillary of the benchmark: four modes, 2^14 samples, 128 nodes.
+        dict(name="capillary_march", kind="capillary_march", n_t=16384, modes=4, nodes=128,
+             raman=0.0, integration="band", absorber="none", attempts=60),
+        # A molecular gas in few modes on an odd radial rule, one probe trial: the Raman
+        # passes over every node and a ragged node count.
+        dict(name="molecular_trial", kind="capillary_trial", n_t=8192, modes=3, nodes=61,
+             raman=0.4, integration="trapezoid", absorber="in_stage", dz=1e-4),
+        # The free-space radial beam of the benchmark: a 512-point Hankel transform.
+        dict(name="radial_march", kind="radial_march", n_t=8192, n_r=512, collar=False,
+             raman=0.0, attempts=32),
+        # A smaller aperture sampled by a number that fits no tile, with its transverse
+        # collar: one probe trial.
+        dict(name="radial_ragged_trial", kind="radial_trial", n_t=4096, n_r=203, collar=True,
+             raman=0.0, dz=1e-4),
+        # The capillary under the fixed schedule of the low-storage replay.
+        dict(name="capillary_replay", kind="replay", n_t=16384, modes=4, nodes=128,
+             schedule=400, steps=16),
+        # A Kerr beam through 12 um of silica on a Cartesian grid with unlike axes.
+        dict(name="beam_replay", kind="beam", nx=256, ny=128, n_t=512, steps=24),
+        # A parameter scan's uneven instances in one batched march.
+        dict(name="scan_rounds", kind="scan", instances=48, draw=3, rounds=16),
+        # The surrogate's training on its own shape, and its screening of scan points.
+        dict(name="surrogate_train", kind="train", width=64, modes=64, layers=4, hidden=128,
+             n=2048, rows=512, batch=64, epochs=2),
+        dict(name="surrogate_screen", kind="screen", width=64, modes=64, layers=4, hidden=128,
+             n=2048, rows=1000, batch=64),
+    ]
+
+
+def draw(rng):
+    def spread(lo, hi):
+        return math.exp(rng.uniform(math.log(lo), math.log(hi)))
+
+    def power(lo, hi):
+        return 1 << rng.randint(lo, hi)
+
+    kind = rng.choice(["envelope_march", "envelope_trial", "session", "capillary_march",
+                       "capillary_trial", "radial_march", "radial_trial", "replay", "beam",
+                       "scan", "train", "screen"])
+    case = {"kind": kind}
+    if kind == "envelope_march":
+        case.update(n_t=power(9, 14), ffac=2, soliton=round(rng.uniform(1.0, 6.0), 2),
+                    absorber=rng.choice(["none", "none", "in_stage", "split_step"]),
+                    noise=rng.choice(["input", "modified", "none"]),
+                    attempts=rng.randint(10, 40))
+    elif kind == "envelope_trial":
+        case.update(n_t=power(9, 16), ffac=rng.choice([1, 2, 2]),
+                    soliton=round(rng.uniform(1.0, 8.0), 2),
+                    absorber=rng.choice(["none", "in_stage"]),
+                    noise=rng.choice(["input", "modified", "none"]),
+                    dz=round(spread(5e-5, 5e-4), 7))
+    elif kind == "session":
+        case.update(n_t=power(11, 13), modes=rng.randint(1, 2), nodes=rng.randint(12, 48),
+                    pressure=round(rng.uniform(0.2, 3.0), 3), energy=spread(20e-6, 300e-6),
+                    fwhm=rng.uniform(5e-15, 30e-15), observations=rng.randint(2, 6), every=8)
+    elif kind in ("capillary_march", "capillary_trial"):
+        case.update(n_t=power(11, 14), modes=rng.randint(1, 6), nodes=rng.randint(16, 128),
+                    raman=rng.choice([0.0, 0.0, 0.3]),
+                    integration=rng.choice(["band", "band", "trapezoid"]),
+                    absorber=rng.choice(["none", "none", "in_stage"]))
+        if case["raman"] and case["n_t"] * case["nodes"] > 2**19:
+            case["n_t"] = 4096
+        if kind == "capillary_march":
+            case["attempts"] = rng.randint(15, 60)
+        else:
+            case["dz"] = round(spread(5e-5, 3e-4), 7)
+    elif kind in ("radial_march", "radial_trial"):
+        case.update(n_t=power(10, 13), n_r=int(spread(12, 512)),
+                    collar=rng.random() < 0.3, raman=0.0)
+        if kind == "radial_march":
+            case["attempts"] = rng.randint(8, 32)
+        else:
+            case["dz"] = round(spread(5e-5, 2e-4), 7)
+    elif kind == "replay":
+        case.update(n_t=power(11, 14), modes=rng.randint(1, 6), nodes=rng.randint(16, 128),
+                    schedule=rng.randint(400, 800), steps=rng.randint(4, 16))
+    elif kind == "beam":
+        case.update(nx=power(4, 8), ny=power(4, 7), n_t=power(6, 9), steps=rng.randint(4, 24))
+    elif kind == "scan":
+        case.update(instances=int(spread(6, 48)), draw=rng.randint(10, 10**6),
+                    rounds=rng.randint(6, 16))
+    else:
+        case.update(width=rng.choice([16, 32, 48, 64]), modes=rng.choice([8, 16, 24, 64]),
+                    layers=rng.randint(2, 4), hidden=rng.choice([32, 64, 128]),
+                    n=rng.choice([256, 500, 1024, 2048]), batch=int(spread(7, 64)))
+        if kind == "train":
+            case.update(rows=case["batch"] * rng.randint(2, 8), epochs=1)
+        else:
+            case.update(rows=int(spread(30, 1000)))
+    return case
+
+
+# --------------------------------------------------------------------------- problems
+
+
+def _band(n_t):
+    """The capillary's wavelength band: a coarser grid resolves a narrower one."""
+    return ({2048: 300e-9, 4096: 200e-9, 8192: 200e-9}.get(n_t, 100e-9), 4e-6)
+
+
+@functools.lru_cache(maxsize=4)
+def _problem(key):
+    c = dict(key)
+    kind = c["kind"]
+    if kind.startswith("envelope"):
+        # The window keeps the builder's sample spacing as the grid grows.
+        return gnlse_problem(n_t=c["n_t"], ffac=c["ffac"], window=10e-12 * c["n_t"] / 8192,
+                             soliton_order=c["soliton"], absorber=c["absorber"],
+                             noise_model=c["noise"])
+    if kind == "session":
+        return capillary_problem(n_t=c["n_t"], window=400e-15 * c["n_t"] / 4096, n_modes=c["modes"],
+                                 n_nodes=c["nodes"], band=surrogate.GRID["band"],
+                                 p0=c["pressure"], p1=c["pressure"], energy=c["energy"],
+                                 fwhm=c["fwhm"])
+    if kind.startswith("capillary"):
+        return capillary_problem(n_t=c["n_t"], n_modes=c["modes"], n_nodes=c["nodes"],
+                                 raman_share=c["raman"], raman_drive="real",
+                                 integration=c["integration"], absorber=c["absorber"],
+                                 band=_band(c["n_t"]))
+    if kind == "replay":
+        p = capillary_problem(n_t=c["n_t"], n_modes=c["modes"], n_nodes=c["nodes"],
+                              band=_band(c["n_t"]))
+        edges = np.linspace(0.0, p.z_end, c["schedule"] + 1)
+        return dataclasses.replace(p, method="low_storage", schedule=edges)
+    if kind.startswith("radial"):
+        large = c["n_t"] >= 4096
+        return radial_problem(n_t=c["n_t"], window=c["n_t"] * (1.0e-12 if large else 2.0e-12) / 8192,
+                              n_r=c["n_r"], fwhm=60e-15 if large else 30e-15,
+                              band=(200e-9 if large else 400e-9, 4e-6),
+                              raman_share=c["raman"],
+                              collar=(1.0e-3, 200.0) if c["collar"] else None)
+    assert kind == "beam"
+    return cartesian_problem(nx=c["nx"], ny=c["ny"], n_t=c["n_t"],
+                             spacing=1.05e-6 * 384 / c["nx"], steps=c["steps"],
+                             length=0.5e-6 * c["steps"])
+
+
+@functools.lru_cache(maxsize=2)
+def _scan_problems(n, seed):
+    """The benchmark's scan: pressure 0.2-3 bar, energy 20-500 uJ, FWHM 5-30 fs, length
+    0.5-3 m, 2^12, 2^13 or 2^14 samples and 1-6 modes."""
+    rng = np.random.default_rng(seed)
+    out = []
+    for _ in range(n):
+        t = int(rng.choice([2**12, 2**13, 2**14]))
+        p = float(rng.uniform(0.2, 3.0))
+        out.append(capillary_problem(
+            n_t=t, window=t * SCAN_DT, n_modes=int(rng.integers(1, 7)), p0=p, p1=p,
+            energy=float(np.exp(rng.uniform(np.log(20e-6), np.log(500e-6)))),
+            fwhm=float(rng.uniform(5e-15, 30e-15)), length=float(rng.uniform(0.5, 3.0))))
+    return out
+
+
+def _key(case):
+    return tuple(sorted((k, v) for k, v in case.items()
+                        if k not in ("name", "attempts", "dz", "observations", "every")
+                        and not (k == "steps" and case["kind"] == "replay")))
+
+
+def _launch(problem, rng):
+    """The builder's launch pulse at another energy (5 %) with another small chirp, as two
+    shots or two scan points differ."""
+    spectrum = np.abs(problem.field0).sum(axis=0)
+    centre = float((spectrum * problem.omega).sum() / spectrum.sum())
+    width = math.sqrt(float((spectrum * (problem.omega - centre) ** 2).sum() / spectrum.sum()))
+    phase = rng.uniform(-0.3, 0.3) * ((problem.omega - centre) / width) ** 2
+    turn = (1.0 + rng.uniform(-0.05, 0.05)) * np.exp(1j * np.where(problem.active_mask, phase, 0.0))
+    return problem.field0 * turn[None, :]
+
+
+def _network(case):
+    shape = surrogate.Shape(width=case["width"], modes=case["modes"], layers=case["layers"],
+                            hidden=case["hidden"], n=case["n"])
+    return shape, surrogate.Network(shape, max_batch=case["batch"])
+
+
+def _parameters(case, rng):
+    """Initial parameters at the network's own scales, in its flat order."""
+    w, m, h = case["width"], case["modes"], case["hidden"]
+    i = surrogate.Shape().in_ch
+
+    def uniform(count, bound):
+        return rng.uniform(-bound, bound, count).astype(np.float32)
+
+    parts = [uniform(w * i, i**-0.5), uniform(w, i**-0.5)]
+    for _ in range(case["layers"]):
+        parts += [uniform(m * w * w, 1.0 / w), uniform(m * w * w, 1.0 / w),
+                  uniform(w * w, w**-0.5), uniform(w, w**-0.5)]
+    parts += [uniform(h * w, w**-0.5), uniform(h, w**-0.5), uniform(h, h**-0.5),
+              uniform(1, h**-0.5)]
+    return np.concatenate(parts)
+
+
+def _rows(case, rng):
+    """Launch spectra of drawn scan points in the network's units, their normalised
+    parameters and an exit change that broadens with energy and pressure."""
+    n = case["n"]
+    points = surrogate.draw(case["rows"], rng)
+    spectra = np.ascontiguousarray(surrogate.launch_log_spectra(points[:, 2])[:, :n])
+    params = surrogate.normalise(points)
+    grid = np.arange(n) / n
+    centre = 0.15 + 0.4 * params[:, :1] * params[:, 1:2]
+    targets = (0.5 * params[:, 1:2] * np.exp(-((grid - centre) / (0.05 + 0.1 * params[:, 3:4])) ** 2)
+               - 0.1 * spectra).astype(np.float32)
+    return spectra, params, targets
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    rng = np.random.default_rng([seed, 17])
+    if kind in ("train", "screen"):
+        shape, net = _network(case)
+        flat = _parameters(case, rng)
+        spectra, params, targets = _rows(case, rng)
+        net.set_parameters(flat)
+        if kind == "train":
+            net.load_dataset(spectra, params, targets)
+        return dict(case=case, net=net, flat=flat, spectra=spectra, params=params,
+                    targets=targets, order=int(rng.integers(1 << 30)))
+    if kind == "scan":
+        problems = _scan_problems(case["instances"], case["draw"])
+        fields = [_launch(p, rng) for p in problems]
+        return dict(case=case, scan=Scan(problems), problems=problems, fields=fields,
+                    targets=np.array([p.z_end for p in problems]))
+    problem = _problem(_key(case))
+    return dict(case=case, problem=problem, ws=Workspace(problem), field=_launch(problem, rng))
+
+
+# -------------------------------------------------------------------------------- run
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "train":
+        net = state["net"]
+        net.set_parameters(state["flat"])
+        losses, _ = net.train(epochs=case["epochs"], batch=case["batch"], seed=state["order"])
+        return {"losses": losses, "parameters": net.parameters()}
+    if kind == "screen":
+        return {"spectra": surrogate.predict(state["net"], state["spectra"], state["params"])}
+    if kind == "scan":
+        scan = state["scan"]
+        for i, field in enumerate(state["fields"]):
+            scan.load(i, 0.0, field)
+        batches = scan.advance(state["targets"], work_limit=case["rounds"])
+        return {"rows": np.concatenate([b.attempts for b in batches]),
+                "fields": np.concatenate([scan.state(i).ravel() for i in range(len(scan))])}
+    ws, problem, field = state["ws"], state["problem"], state["field"]
+    if kind.endswith("_trial"):
+        probe = ws.probe(0.0, field)
+        norm = probe.trial(0.0, case["dz"])
+        return {"field": probe.field(), "norm": np.float64(norm)}
+    if kind == "session":
+        return _session(case, ws, problem, field)
+    march = ws.march(0.0, field)
+    if kind in ("replay", "beam"):
+        edge = float(problem.schedule[case["steps"]])
+        rows = march.run(edge)
+    else:
+        rows = march.advance(problem.z_end, work_limit=case["attempts"]).attempts
+    return {"field": march.state(), "rows": rows}
+
+
+def _session(case, ws, problem, field):
+    session = ws.start({"z": 0.0, "field": field, "planes": [problem.z_end], "launch": False,
+                        "step_planes": case["every"],
+                        "statistics": ["energy", "peak_power", "electron_density"]})
+    rows, stats = [], []
+    for seen in range(case["observations"]):
+        batch = session.advance(100000, 100.0)
+        rows.append(batch.attempts[:, :5])  # the sixth column is wall time
+        stats.append(batch.plane_stats)
+        if seen == case["observations"] - 1:
+            out = np.empty((problem.n_modes, problem.n_omega), dtype=np.complex128)
+            session.export(batch.ticket, {"power_weight": None, "optics": True}, out)
+        session.acknowledge(batch.sequence)
+    session.close()
+    return {"rows": np.concatenate(rows), "stats": np.stack(stats), "field": out}
+
+
+# ------------------------------------------------------------------------------- work
+
+
+def _field_attempt(c, n, t, q, stored, phi, streams):
+    """One source evaluation and its Adams or replay arithmetic: the state, the operator
+    and prefactor rows and the stored source rows read once, the state and the newest
+    source written; the transforms, the products over the nodes and the responses."""
+    bytes_ = 16.0 * c * n * (1 + phi + 1 + stored + 2) + 8.0 * 2 * q * c
+    fft = 2.5 * t * math.log2(t) * c * (1 + streams)
+    nodes = 2.0 * q * c * t * (1 + min(streams, 2)) + 60.0 * q * t
+    return bytes_, fft + nodes + 60.0 * c * n
+
+
+def work(case):
+    kind = case["kind"]
+    if kind in ("train", "screen"):
+        w, m, n, h, ell = (case[k] for k in ("width", "modes", "n", "hidden", "layers"))
+        forward = 2.0 * (ell * (2 * w * n * 2 * m + w * w * n + 4 * m * w * w) + h * w * n)
+        count = 4.0 * (w * 7 + ell * (2 * m * w * w + w * w + w) + h * w + 2 * h + 1)
+        if kind == "screen":
+            return {"bytes": count + 4.0 * case["rows"] * (2 * n + 4),
+                    "flops": forward * case["rows"]}
+        steps = case["epochs"] * (case["rows"] // case["batch"])
+        # A step reads the batch, and reads and writes the parameters and two moments.
+        return {"bytes": steps * (4.0 * case["batch"] * (2 * n + 4) + 6 * count),
+                "flops": 3.0 * forward * case["batch"] * steps}
+    if kind == "scan":
+        total = {"bytes": 0.0, "flops": 0.0}
+        for p in _scan_problems(case["instances"], case["draw"]):
+            b, f = _field_attempt(p.n_modes, p.n_omega, p.n_to, p.n_nodes, 4, 2, 3)
+            total["bytes"] += case["rounds"] * b
+            total["flops"] += case["rounds"] * f
+        return total
+    if kind == "beam":
+        points = case["nx"] * case["ny"] * case["n_t"]
+        fft = 5.0 * points * math.log2(points)
+        return {"bytes": case["steps"] * 16.0 * points * 4,
+                "flops": case["steps"] * (8 * fft + 150.0 * points)}
+    if kind.startswith("envelope"):
+        t = case["n_t"] * case["ffac"]
+        # A stage: the coarse state, operator and prefactor, and the stage rows; two
+        # transforms of the fine grid and two real ones of the doubled grid.
+        stages = 6 * case["attempts"] if kind == "envelope_march" else 7
+        fft = 5.0 * t * math.log2(t) * 2 + 2.5 * 2 * t * math.log2(2 * t) * 2
+        return {"bytes": stages * (16.0 * case["n_t"] * 6 + 16.0 * t),
+                "flops": stages * (fft + 100.0 * case["n_t"] + 30.0 * t)}
+    if kind.startswith("radial"):
+        c, n, q, t = case["n_r"], case["n_t"] // 2 + 1, case["n_r"], case["n_t"]
+        attempts = case["attempts"] if kind == "radial_march" else 2
+        b, f = _field_attempt(c, n, t, q, 4 if kind == "radial_march" else 1, 1, 3)
+        return {"bytes": attempts * b, "flops": attempts * f}
+    c, n, q, t = case["modes"], case["n_t"] // 2 + 1, case["nodes"], case["n_t"]
+    if kind == "replay":
+        attempts, stored = 4 * case["steps"], 1
+    elif kind == "session":
+        attempts, stored = case["observations"] * case["every"], 4
+    elif kind == "capillary_march":
+        attempts, stored = case["attempts"], 4
+    else:
+        attempts, stored = 2, 1
+    b, f = _field_attempt(c, n, t, q, stored, 2, 3)
+    if case.get("raman"):
+        f += q * 2 * 2.5 * 2 * t * math.log2(2 * t)
+    return {"bytes": attempts * b, "flops": attempts * f}
+
+
+def tolerance(case):
+    """About four times what a build without fused multiply-adds and a launch moved by one
+    unit in the last place were measured to change, or what 64 bits say, whichever is more."""
+    kind = case["kind"]
+    if kind == "train":
+        return {"rel": 4.4e-3, "max": 0.7}  # bf16 products; Adam divides by small moments
+    if kind == "screen":
+        return {"rel": 1.2e-3, "max": 6e-3}
+    if kind in ("replay", "beam"):
+        return {"rel": 1.2e-14}
+    if kind.endswith("_trial"):
+        return {"rel": 4e-9}  # the norm is an error estimate that cancels; fields hold 1e-15
+    return {"rel": 5e-10}  # step sizes follow the norms
+
+
+# ------------------------------------------------- the same in 64 bits, in plain torch
+
+
+def _device():
+    return "cuda" if torch.cuda.is_available() else "cpu"
+
+
+def _t(a, dtype=torch.float64):
+    return torch.as_tensor(np.ascontiguousarray(a), device=_device()).to(dtype)
+
+
+def _c(a):
+    return _t(a, torch.complex128)
+
+
+def _path(p, z, derivative=False):
+    """A scalar path at z: a constant, the position, or a Chebyshev series on its piece."""
+    if p.kind == 0:
+        return 0.0 if derivative else float(p.value)
+    if p.kind == 1:
+        return 1.0 if derivative else float(z)
+    j = min(max(int(np.searchsorted(p.edges, z, side="right")) - 1, 0), len(p.edges) - 2)
+    a, b = p.edges[j], p.edges[j + 1]
+    series = np.polynomial.chebyshev.Chebyshev(p.coefficients[j], domain=[a, b])
+    return float((series.deriv() if derivative else series)(z))
+
+
+class _Source:
+    """The nonlinear source of a problem at a lab-frame spectrum, (C, N)."""
+
+    def __init__(self, p):
+        self.p = p
+        self.real = p.kind == "field"
+        self.phi = [_c(term) for term in p.phi_terms]
+        self.pref = [_c(term) for term in p.prefactor_terms]
+        self.window = _t(p.omega_window)
+        self.active = _t(p.active_mask)
+        self.crop = torch.as_tensor(p.crop_index, device=_device())
+        self.collar, self.collar_rate = _t(p.time_window), _t(p.time_window_derivative)
+        self.up, self.down = _t(p.synthesis), _t(p.projection)
+        self.absorber = _t(p.absorber_rate) if p.absorber_scheme == "in_stage" else None
+        self.spatial = None if p.spatial_absorber is None else _t(p.spatial_absorber)
+
+    def operator(self, z0, z1):
+        return sum((_path(w, z1) - _path(w, z0)) * term
+                   for w, term in zip(self.p.phi_paths, self.phi))
+
+    def operator_rate(self, z):
+        return sum(_path(w, z, True) * term for w, term in zip(self.p.phi_paths, self.phi))
+
+    def cumulative(self, y, filtered):
+        """The running trapezoid along time, of the symmetrically filtered samples."""
+        taps = [float(v) for v in self.p.plasma.taps]
+        half = len(taps) - 1
+        f = y
+        if filtered and half:
+            head = 2.0 * y[:, :1] - y[:, 1:half + 1].flip(1)
+            tail = 2.0 * y[:, -1:] - y[:, -half - 1:-1].flip(1)
+            e = torch.cat([head, y, tail], dim=1)
+            n = y.shape[1]
+            f = taps[0] * y
+            for k in range(1, half + 1):
+                f = f + taps[k] * (e[:, half - k:half - k + n] + e[:, half + k:half + k + n])
+        step = 0.5 * self.p.dt_fine * (f[:, 1:] + f[:, :-1])
+        return torch.cat([torch.zeros_like(f[:, :1]), torch.cumsum(step, dim=1)], dim=1)
+
+    def rate(self, e):
+        g = self.p.plasma
+        size = e.abs()
+        log = torch.log(size.clamp_min(1e-300))
+        coefficients = _t(g.rate_coefficients)
+        at = ((log - g.log_field_min) / g.d_log_field).floor().long()
+        at = at.clamp(0, coefficients.shape[1] - 1)
+        u = log - (g.log_field_min + at.double() * g.d_log_field)
+        k = [coefficients[i][at] for i in range(4)]
+        w = torch.exp(((k[0] * u + k[1]) * u + k[2]) * u + k[3])
+        w = torch.where(size < g.field_min, torch.zeros_like(w), w)
+        return torch.where(size > g.field_max, torch.full_like(w, g.rate_max), w)
+
+    def current(self, e, z):
+        g = self.p.plasma
+        w = self.rate(e)
+        exposure = self.cumulative(w, True)
+        if len(g.taps) > 1:
+            exposure = exposure.clamp_min(0.0)
+        freed = 1.0 - (1.0 - _path(self.p.preionisation, z)) * torch.exp(-exposure)
+        free = self.cumulative(freed * g.charge_mass_ratio * e, True)
+        loss = torch.where((w > 0) & (e != 0), g.ionisation_potential * w * (1.0 - freed)
+                           / torch.where(e != 0, e, torch.ones_like(e)), torch.zeros_like(e))
+        return _path(self.p.density, z) * (free + loss)
+
+    def delayed(self, e, z):
+        """The Raman term: the drive convolved with the damped response over the past."""
+        r, p, t = self.p.raman, self.p, e.shape[-1]
+        delay = torch.arange(2 * t, device=e.device, dtype=torch.float64) * p.dt_fine
+        kernel = sum(_t(row) * torch.exp(-_path(w, z) * delay)
+                     for row, w in zip(r.undamped, r.rates))
+        spectrum = torch.fft.rfft(r.fraction * kernel) * p.dt_fine
+        if not self.real:
+            drive = 0.5 * e.abs() ** 2
+        elif r.thg:
+            drive = e**2
+        else:
+            gain = torch.full((t,), 2.0, device=e.device, dtype=torch.float64)
+            gain[0] = gain[t // 2] = 1.0
+            gain[t // 2 + 1:] = 0.0
+            drive = 0.5 * torch.fft.ifft(torch.fft.fft(e) * gain).abs() ** 2
+        out = torch.fft.irfft(spectrum * torch.fft.rfft(drive, n=2 * t), n=2 * t)[..., :t]
+        return r.epsilon0 * _path(p.density, z) * e * out
+
+    def __call__(self, lab, z):
+        p = self.p
+        t = p.n_to
+        if self.real:
+            modal = torch.fft.irfft(lab, n=t)
+        else:
+            fine = torch.zeros((lab.shape[0], t), dtype=lab.dtype, device=lab.device)
+            fine[:, self.crop] = lab
+            modal = torch.fft.ifft(fine)
+        e = self.up.to(modal.dtype) @ modal
+        local = torch.zeros_like(e)
+        if p.kerr is not None:
+            k, scale = p.kerr, p.kerr.coefficient * _path(p.density, z)
+            if k.cubic_form == "real":
+                local = local + scale * e**3
+            else:
+                local = local + scale * (k.self_factor * e.abs() ** 2 * e
+                                         + k.conjugate_factor * e**2 * e.conj())
+        if p.raman is not None:
+            local = local + self.delayed(e, z)
+        transform = torch.fft.rfft if self.real else torch.fft.fft
+        down = self.down.to(modal.dtype)
+        out = transform(down @ (self.collar * local))[:, self.crop]
+        if p.plasma is not None:
+            j = down @ self.current(e, z)
+            omega = torch.where(self.active > 0, _t(p.omega), torch.ones_like(self.active))
+            held = (transform(self.collar * j)[:, self.crop] / (1j * omega)
+                    + transform(self.collar_rate * j)[:, self.crop] / omega**2)
+            out = out + held * self.active
+        out = out * self.window * sum(_path(w, z) * term
+                                      for w, term in zip(p.prefactor_paths, self.pref))
+        extra = None
+        if self.absorber is not None:
+            extra = -0.5 * self.absorber * modal
+        if self.spatial is not None:
+            extra = self.spatial @ modal + (0.0 if extra is None else extra)
+        if extra is not None:
+            out = out + transform(extra)[:, self.crop] * self.active
+        return out
+
+
+class _BeamSource:
+    """The Kerr source of a Cartesian envelope, (C, N) on columns iy nx + ix."""
+
+    def __init__(self, p):
+        self.p = p
+        nx, ny = p.transverse
+        self.grid = (ny, nx, p.n_t)
+        self.phi, self.pref = _c(p.phi_terms[0]), _c(p.prefactor_terms[0])
+
+    def operator(self, z0, z1):
+        return (z1 - z0) * self.phi
+
+    def __call__(self, lab, z):
+        k = self.p.kerr
+        e = torch.fft.ifftn(lab.reshape(self.grid))
+        e = (k.coefficient * k.self_factor) * e.abs() ** 2 * e
+        return self.pref * torch.fft.fftn(e).reshape(lab.shape)
+
+
+def _phi_two(x):
+    """(phi_1, phi_2) of a complex argument: the series inside the unit disc."""
+    near = x.abs() < 1.0
+    y = torch.where(near, x, torch.zeros_like(x))
+    far = torch.where(near, torch.ones_like(x), x)
+    s1, s2 = torch.zeros_like(x), torch.zeros_like(x)
+    for k in range(24, -1, -1):
+        s1 = s1 * y + 1.0 / math.factorial(k + 1)
+        s2 = s2 * y + 1.0 / math.factorial(k + 2)
+    f1 = (torch.exp(far) - 1.0) / far
+    f2 = (f1 - 1.0) / far
+    return torch.where(near, s1, f1), torch.where(near, s2, f2)
+
+
+def _adams_trial(p, y, dz):
+    """The first exponential Adams trial from z = 0: one stored source, order one."""
+    source = _Source(p)
+    x = source.operator(0.0, dz)
+    flow = torch.exp(x)
+    m0, m1 = _phi_two(x)
+    s0 = source(y, 0.0)
+    lab = flow * y + dz * m0 * s0
+    carried = None
+    if len(p.phi_paths) > 1:  # the operator varies: its part off the step's mean rate
+        carried = flow * ((source.operator_rate(0.0) - x / dz) * y)
+        lab = lab + dz * carried
+    s1 = source(lab, dz)
+    advanced = flow * y + dz * (m0 * s0 + m1 * (s1 - s0))
+    defect = dz * m1 * (s1 - s0)
+    if carried is not None:
+        end = (source.operator_rate(dz) - x / dz) * lab
+        advanced = advanced + 0.5 * dz * (end + carried)
+        defect = defect + 0.5 * dz * (end - carried)
+    mask = torch.as_tensor(p.norm_mask, device=y.device)
+    scale = p.rtol * float(torch.linalg.norm(y[:, mask])) + p.atol
+    return {"field": advanced.cpu().numpy(),
+            "norm": np.float64(float(torch.linalg.norm(defect[:, mask])) / scale)}
+
+
+def _runge_kutta_trial(p, y, dz):
+    """One interaction-picture trial of the embedded pair from z = 0."""
+    source, tab = _Source(p), p.tableau
+    noise = None
+    if p.noise_model == "modified" and p.noise0 is not None:
+        noise = _c(p.noise0)
+    stages = []
+    for i, node in enumerate(tab.nodes):
+        x = source.operator(0.0, float(node) * dz)
+        lab = y + dz * sum((float(tab.matrix[i, j]) * stages[j] for j in range(i)),
+                           torch.zeros_like(y))
+        lab = torch.exp(x) * lab
+        if noise is not None:
+            turned = sum(_path(w, float(node) * dz) * term
+                         for w, term in zip(p.phi_paths, source.phi))
+            lab = lab + noise * torch.exp(1j * turned.imag)
+        stages.append(torch.exp(-x) * source(lab, float(node) * dz))
+    flow = torch.exp(source.operator(0.0, dz))
+    advanced = flow * (y + dz * sum(float(b) * k for b, k in zip(tab.solution_weights, stages)))
+    error = flow * dz * sum(float(w) * k for w, k in zip(tab.error_weights, stages))
+    mask = torch.as_tensor(p.norm_mask, device=y.device)
+    scale = p.rtol * max(float(torch.linalg.norm(y[:, mask])),
+                         float(torch.linalg.norm(advanced[:, mask]))) + p.atol
+    return {"field": advanced.cpu().numpy(),
+            "norm": np.float64(float(torch.linalg.norm(error[:, mask])) / scale)}
+
+
+def _replay(p, y, steps):
+    """Fixed fourth-order interaction-picture steps over the schedule's first edges."""
+    source = _BeamSource(p) if p.kind == "cartesian" else _Source(p)
+    mask = torch.as_tensor(p.active_mask, device=y.device)
+    rows = []
+    for i in range(steps):
+        z0, z1 = float(p.schedule[i]), float(p.schedule[i + 1])
+        dz = z1 - z0
+        mid = z0 + 0.5 * dz
+        first = torch.exp(source.operator(z0, mid))
+        second = torch.exp(source.operator(mid, z0 + dz))
+        moved = first * y
+        k1 = first * source(y, z0)
+        k2 = source(moved + 0.5 * dz * k1, mid)
+        k3 = source(moved + 0.5 * dz * k2, mid)
+        k4 = source(second * (moved + dz * k3), z0 + dz)
+        y = second * (moved + dz / 6.0 * (k1 + 2.0 * k2 + 2.0 * k3)) + dz / 6.0 * k4
+        y = y * mask
+        rows.append((z1, dz, 0.0, 1.0))
+    return {"field": y.cpu().numpy(), "rows": np.array(rows)}
+
+
+def _tensors(case, flat):
+    """The network's parameters by name from the flat vector, as 64-bit leaves."""
+    w, m, h = case["width"], case["modes"], case["hidden"]
+    i = surrogate.Shape().in_ch
+    shapes = [(w, i), (w,)]
+    for _ in range(case["layers"]):
+        shapes += [(m, w, w), (m, w, w), (w, w), (w,)]
+    shapes += [(h, w), (h,), (h,), (1,)]
+    out, at = [], 0
+    for shape in shapes:
+        size = math.prod(shape)
+        out.append(_t(flat[at:at + size]).reshape(shape).requires_grad_())
+        at += size
+    return out
+
+
+def _infer(case, weights, spectra, params):
+    """The network's output: a lift, Fourier layers over the kept modes, a head."""
+    m, n = case["modes"], case["n"]
+    grid = (torch.arange(n, device=spectra.device, dtype=torch.float64) / n).expand_as(spectra)
+    x = torch.stack([spectra, *[c[:, None].expand_as(spectra) for c in params.unbind(1)], grid],
+                    dim=1)
+    v = weights[0] @ x + weights[1][:, None]
+    for layer in range(case["layers"]):
+        re, im, w, b = weights[2 + 4 * layer:6 + 4 * layer]
+        kept = torch.fft.rfft(v)[..., :m].permute(2, 0, 1)
+        mixed = torch.bmm(kept.contiguous(), torch.complex(re, im)).permute(1, 2, 0)
+        z = torch.fft.irfft(mixed, n=n) + w @ v + b[:, None]
+        last = layer == case["layers"] - 1
+        v = z if last else torch.nn.functional.gelu(z, approximate="tanh")
+    q1, b1, q2, b2 = weights[-4:]
+    hidden = torch.nn.functional.gelu(q1 @ v + b1[:, None], approximate="tanh")
+    return (q2[:, None] * hidden).sum(dim=1) + b2
+
+
+def _train(case, state):
+    weights = _tensors(case, state["flat"])
+    first = [torch.zeros_like(w) for w in weights]
+    second = [torch.zeros_like(w) for w in weights]
+    spectra, params, targets = (_t(state[k]) for k in ("spectra", "params", "targets"))
+    rng = np.random.default_rng(state["order"])
+    per = case["rows"] // case["batch"]
+    order = np.concatenate([rng.permutation(case["rows"])[:per * case["batch"]]
+                            for _ in range(case["epochs"])])
+    losses = []
+    for step, rows in enumerate(order.reshape(-1, case["batch"]), start=1):
+        rows = torch.as_tensor(rows, device=spectra.device)
+        loss = ((_infer(case, weights, spectra[rows], params[rows]) - targets[rows]) ** 2).mean()
+        grads = torch.autograd.grad(loss, weights)
+        size = 1e-3 * math.sqrt(1.0 - 0.999**step) / (1.0 - 0.9**step)
+        with torch.no_grad():
+            for w, g, m, v in zip(weights, grads, first, second):
+                m.mul_(0.9).add_(g, alpha=0.1)
+                v.mul_(0.999).addcmul_(g, g, value=0.001)
+                w.sub_(size * m / (v.sqrt() + 1e-8))
+        losses.append(float(loss.detach()))
+    flat = torch.cat([w.detach().reshape(-1) for w in weights])
+    return {"losses": np.array(losses), "parameters": flat.cpu().numpy()}
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind in ("train", "screen"):
+        rng = np.random.default_rng([seed, 17])
+        flat = _parameters(case, rng)
+        spectra, params, targets = _rows(case, rng)
+        if kind == "train":
+            return _train(case, dict(flat=flat, spectra=spectra, params=params, targets=targets,
+                                     order=int(rng.integers(1 << 30))))
+        weights = _tensors(case, flat)
+        out = []
+        with torch.no_grad():
+            for a, b in zip(_t(spectra).split(64), _t(params).split(64)):
+                out.append(a + _infer(case, weights, a, b))
+        return {"spectra": torch.cat(out).cpu().numpy()}
+    if kind not in ("replay", "beam") and not kind.endswith("_trial"):
+        return None  # an adaptive march: its steps are its controller's own
+    problem = _problem(_key(case))
+    y = _c(_launch(problem, np.random.default_rng([seed, 17])))
+    if kind == "envelope_trial":
+        return _runge_kutta_trial(problem, y, case["dz"])
+    if kind.endswith("_trial"):
+        return _adams_trial(problem, y, case["dz"])
+    return _replay(problem, y, case["steps"])
