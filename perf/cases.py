@@ -327,7 +327,11 @@ def _session(case, ws, problem, field):
             session.export(batch.ticket, {"power_weight": None, "optics": True}, out)
         session.acknowledge(batch.sequence)
     session.close()
-    return {"rows": np.concatenate(rows), "stats": np.stack(stats), "field": out}
+    # The log of attempts, the tail of its buffer unused (rejected attempts are few).
+    log = np.zeros((2 * case["observations"] * case["every"], 5))
+    rows = np.concatenate(rows)[:len(log)]
+    log[:len(rows)] = rows
+    return {"rows": log, "stats": np.stack(stats), "field": out}
 
 
 # ------------------------------------------------------------------------------- work
