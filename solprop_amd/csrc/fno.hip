@@ -1,6 +1,7 @@
 // The learned surrogate's kernels (see fno.hpp): BF16 matrix-core products with fused
 // epilogues, the spectral mixing, the head, the loss, reductions and Adam.
 #include "fno.hpp"
+#include "fno_tile.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -474,7 +475,7 @@ __global__ void lift_backward(const float* __restrict__ dv, const float* __restr
 }
 
 // Adam (Kingma and Ba 2015) with the bias corrections folded into the step size, and
-// the BF16 mirror refreshed.
+// the BF16 mirror, where there is one, refreshed.
 __global__ void adam(float* __restrict__ p, bf16* __restrict__ p16, const float* __restrict__ g,
                      float* __restrict__ m, float* __restrict__ v, long count, float step,
                      float beta1, float beta2, float eps) {
@@ -487,7 +488,7 @@ __global__ void adam(float* __restrict__ p, bf16* __restrict__ p16, const float*
   v[i] = vi;
   const float pi = p[i] - step * mi / (sqrtf(vi) + eps);
   p[i] = pi;
-  p16[i] = to_bf16(pi);
+  if (p16) p16[i] = to_bf16(pi);
 }
 
 __global__ void to_bf16_kernel(const float* __restrict__ x, bf16* __restrict__ y, long count) {
@@ -510,6 +511,26 @@ __global__ void gather(const int* __restrict__ idx, const float* __restrict__ sp
 }
 
 unsigned blocks(long n, int threads) { return static_cast<unsigned>((n + threads - 1) / threads); }
+
+
+// The truncated transforms F (n, 2 modes) and G (2 modes, n), rounded to BF16 on the host
+// from FP64 angles reduced exactly.
+void transforms(const Shape& s, std::vector<bf16>& f, std::vector<bf16>& g) {
+  const long n = s.n, M = s.modes;
+  f.resize(n * 2 * M);
+  g.resize(2 * M * n);
+  const double two_pi = 6.283185307179586;
+  for (long t = 0; t < n; ++t)
+    for (long k = 0; k < M; ++k) {
+      const double a = two_pi * static_cast<double>((t * k) % n) / static_cast<double>(n);
+      const double c = std::cos(a), sn = std::sin(a);
+      const double w = (k == 0 ? 1.0 : 2.0) / static_cast<double>(n);
+      f[t * 2 * M + k] = to_bf16(static_cast<float>(c));
+      f[t * 2 * M + M + k] = to_bf16(static_cast<float>(-sn));
+      g[k * n + t] = to_bf16(static_cast<float>(w * c));
+      g[(M + k) * n + t] = to_bf16(static_cast<float>(-w * sn));
+    }
+}
 
 }  // namespace
 
@@ -561,48 +582,17 @@ Network::Network(const Shape& s, int max_batch) : s_(s), off_(offsets(s)), max_b
     grad_ = alloc<float>(P);
     m_ = alloc<float>(P);
     v_ = alloc<float>(P);
-    param16_ = alloc<bf16>(P);
-    const long n = s.n, M = s.modes, W = s.width, H = s.hidden, B = max_batch;
-    // Transforms, rounded to BF16 on the host from FP64 angles reduced exactly.
-    std::vector<bf16> f(n * 2 * M), g(2 * M * n);
-    const double two_pi = 6.283185307179586;
-    for (long t = 0; t < n; ++t)
-      for (long k = 0; k < M; ++k) {
-        const double a = two_pi * static_cast<double>((t * k) % n) / static_cast<double>(n);
-        const double c = std::cos(a), sn = std::sin(a);
-        const double w = (k == 0 ? 1.0 : 2.0) / static_cast<double>(n);
-        f[t * 2 * M + k] = to_bf16(static_cast<float>(c));
-        f[t * 2 * M + M + k] = to_bf16(static_cast<float>(-sn));
-        g[k * n + t] = to_bf16(static_cast<float>(w * c));
-        g[(M + k) * n + t] = to_bf16(static_cast<float>(-w * sn));
-      }
-    f16_ = alloc<bf16>(f.size());
-    g16_ = alloc<bf16>(g.size());
-    SP_HIP(hipMemcpyAsync(f16_, f.data(), f.size() * 2, hipMemcpyHostToDevice, stream_));
-    SP_HIP(hipMemcpyAsync(g16_, g.data(), g.size() * 2, hipMemcpyHostToDevice, stream_));
+    const long n = s.n, B = max_batch;
     spec_ = alloc<float>(B * n);
     prm_ = alloc<float>(B * std::max(1, s.n_params));
     tgt_ = alloc<float>(B * n);
     out_ = alloc<float>(B * n);
-    for (int l = 0; l <= s.layers; ++l) v16_.push_back(alloc<bf16>(B * W * n));
-    for (int l = 0; l < s.layers; ++l) {
-      z_.push_back(alloc<float>(B * W * n));
-      vhat_.push_back(alloc<float>(B * W * 2 * M));
-    }
-    yhat16_ = alloc<bf16>(B * W * 2 * M);
-    h1_ = alloc<float>(B * H * n);
-    h16_ = alloc<bf16>(B * H * n);
     dout_ = alloc<float>(B * n);
-    dout16_ = alloc<bf16>(B * n);
-    dv_ = alloc<float>(B * W * n);
-    dz_ = alloc<float>(B * W * n);
-    dz16_ = alloc<bf16>(B * W * n);
-    dyhat_ = alloc<float>(B * W * 2 * M);
-    dvhat16_ = alloc<bf16>(B * W * 2 * M);
-    dh1_ = alloc<float>(B * H * n);
-    dh116_ = alloc<bf16>(B * H * n);
     partials_ = alloc<float>(blocks(B * n, 256) + 1);  // the partial sums, then the loss
-    split_ = alloc<float>(kSplitFloats);
+    if (tile_available(s))
+      allocate_tiles();
+    else
+      allocate_general();
     SP_HIP(hipStreamSynchronize(stream_));
   } catch (...) {
     for (void* p : owned_) (void)hipFree(p);
@@ -610,6 +600,146 @@ Network::Network(const Shape& s, int max_batch) : s_(s), off_(offsets(s)), max_b
     if (stream_) (void)hipStreamDestroy(stream_);
     throw;
   }
+}
+
+struct TilePath {
+  TileShape shape;
+  TileBuffers buf;
+};
+
+void Network::allocate_general() {
+  const long n = s_.n, M = s_.modes, W = s_.width, H = s_.hidden, B = max_batch_;
+  param16_ = alloc<bf16>(off_.total);
+  std::vector<bf16> f, g;
+  transforms(s_, f, g);
+  f16_ = alloc<bf16>(f.size());
+  g16_ = alloc<bf16>(g.size());
+  SP_HIP(hipMemcpyAsync(f16_, f.data(), f.size() * 2, hipMemcpyHostToDevice, stream_));
+  SP_HIP(hipMemcpyAsync(g16_, g.data(), g.size() * 2, hipMemcpyHostToDevice, stream_));
+  for (int l = 0; l <= s_.layers; ++l) v16_.push_back(alloc<bf16>(B * W * n));
+  for (int l = 0; l < s_.layers; ++l) {
+    z_.push_back(alloc<float>(B * W * n));
+    vhat_.push_back(alloc<float>(B * W * 2 * M));
+  }
+  yhat16_ = alloc<bf16>(B * W * 2 * M);
+  h1_ = alloc<float>(B * H * n);
+  h16_ = alloc<bf16>(B * H * n);
+  dv_ = alloc<float>(B * W * n);
+  dz_ = alloc<float>(B * W * n);
+  dz16_ = alloc<bf16>(B * W * n);
+  dyhat_ = alloc<float>(B * W * 2 * M);
+  dvhat16_ = alloc<bf16>(B * W * 2 * M);
+  dh1_ = alloc<float>(B * H * n);
+  dh116_ = alloc<bf16>(B * H * n);
+  split_ = alloc<float>(kSplitFloats);
+  SP_HIP(hipStreamSynchronize(stream_));
+}
+
+void Network::allocate_tiles() {
+  tiles_ = std::make_unique<TilePath>();
+  const TileShape t = tiles_->shape = tile_shape(s_);
+  TileBuffers& b = tiles_->buf;
+  const long n = s_.n, M = s_.modes, B = max_batch_, NP = t.NP, WP = t.WP, MP = t.MP;
+  const int L = s_.layers, in_ch = s_.in_ch();
+  std::vector<bf16> f, g;
+  transforms(s_, f, g);
+  // Both tables both ways round, the padded modes and bins zero.
+  std::vector<bf16> table[4];  // g_s, f_k, f_s, g_k
+  for (auto& v : table) v.assign(NP * MP, 0);
+  for (long k = 0; k < 2 * M; ++k) {
+    const long kp = k < M ? k : MP / 2 + k - M;
+    for (long x = 0; x < n; ++x) {
+      table[0][x * MP + kp] = table[3][kp * NP + x] = g[k * n + x];
+      table[1][kp * NP + x] = table[2][x * MP + kp] = f[x * 2 * M + k];
+    }
+  }
+  bf16** to[4] = {&b.g_s, &b.f_k, &b.f_s, &b.g_k};
+  for (int i = 0; i < 4; ++i) {
+    *to[i] = alloc<bf16>(NP * MP);
+    SP_HIP(hipMemcpyAsync(*to[i], table[i].data(), NP * MP * 2, hipMemcpyHostToDevice, stream_));
+  }
+  bf16* w = alloc<bf16>(2 * L * WP * WP);
+  bf16* q = alloc<bf16>(2 * kHeadUnits * WP);
+  b.q1 = q;
+  b.q1t = q + kHeadUnits * WP;
+  const long spectrum = MP * B * WP, groups = tile_groups(max_batch_);
+  float* spectra = alloc<float>(2 * L * spectrum);
+  b.rows = max_batch_;
+  for (int l = 0; l < L; ++l) {
+    b.w.push_back(w + l * WP * WP);
+    b.wt.push_back(w + (L + l) * WP * WP);
+    b.yhat.push_back(alloc<bf16>(spectrum));
+    b.vhat.push_back(spectra + l * spectrum);
+    b.dyhat.push_back(spectra + (L + l) * spectrum);
+    b.dw.push_back(alloc<float>(groups * (WP * WP + WP)));
+  }
+  for (int l = 0; l <= L; ++l) b.v.push_back(alloc<bf16>(B * NP * WP));
+  b.dvhat = alloc<bf16>(spectrum);
+  for (auto& dz : b.dz) dz = alloc<bf16>(B * NP * WP);
+  b.share = alloc<float>(groups * MP * WP);
+  b.dq = alloc<float>(groups * head_share(t.WP));
+  b.dlift = alloc<float>(groups * 3 * WP);
+  b.loss = alloc<float>(groups);
+  // Where each workgroup share of a weight gradient lies, and where its sum goes.
+  std::vector<GradientSegment> seg;
+  int first = 0;
+  auto add = [&](const float* src, long stride, long dst, int rows, int cols, int src_ld,
+                 int dst_ld, int scan_parameter) {
+    seg.push_back({src, stride, grad_ + dst, rows, cols, src_ld, dst_ld, scan_parameter, first});
+    first += (rows * cols + 63) / 64;
+  };
+  const int W = s_.width, H = s_.hidden;
+  const long layer = WP * WP + WP, head = head_share(t.WP);
+  const float* sums = b.dq + kHeadUnits * WP;
+  for (int l = 0; l < L; ++l) {
+    add(b.dw[l], layer, off_.w[l], W, W, t.WP, W, -1);
+    if (l + 1 < L)
+      add(b.dw[l] + WP * WP, layer, off_.b[l], 1, W, t.WP, W, -1);
+    else
+      add(sums + 2 * kHeadUnits, head, off_.b[l], 1, W, t.WP, W, -1);
+  }
+  add(b.dq, head, off_.q1_w, H, W, t.WP, W, -1);
+  add(sums, head, off_.q1_b, 1, H, H, H, -1);
+  add(sums + kHeadUnits, head, off_.q2_w, 1, H, H, H, -1);
+  add(sums + 2 * kHeadUnits + WP, head, off_.q2_b, 1, 1, 1, 1, -1);
+  add(b.dlift, 3 * WP, off_.lift_b, 1, W, t.WP, W, -1);
+  add(b.dlift + WP, 3 * WP, off_.lift_w, W, 1, 1, in_ch, -1);
+  for (int j = 0; j < s_.n_params; ++j)
+    add(b.dlift, 3 * WP, off_.lift_w + 1 + j, W, 1, 1, in_ch, j);
+  add(b.dlift + 2 * WP, 3 * WP, off_.lift_w + 1 + s_.n_params, W, 1, 1, in_ch, -1);
+  b.n_segments = static_cast<int>(seg.size());
+  b.segment_blocks = first;
+  b.segments = alloc<GradientSegment>(seg.size());
+  SP_HIP(hipMemcpyAsync(b.segments, seg.data(), seg.size() * sizeof(GradientSegment),
+                        hipMemcpyHostToDevice, stream_));
+  SP_HIP(hipStreamSynchronize(stream_));
+}
+
+void Network::parameters_changed() {
+  if (tiles_) tile_pack(tiles_->shape, off_, param_, tiles_->buf, stream_);
+}
+
+void Network::run_forward(int batch, float* loss) {
+  if (tiles_) {
+    tile_forward(tiles_->shape, off_, param_, tiles_->buf, spec_, prm_, out_, loss ? tgt_ : nullptr,
+                 dout_, loss, batch, loss != nullptr, stream_);
+    return;
+  }
+  general_forward(batch);
+  if (!loss) return;
+  const long count = static_cast<long>(batch) * s_.n;
+  const unsigned nb = blocks(count, 256);
+  hipLaunchKernelGGL(loss_grad, dim3(nb), dim3(256), 0, stream_, out_, tgt_, dout_, partials_, count);
+  hipLaunchKernelGGL(loss_total, dim3(1), dim3(256), 0, stream_, partials_, static_cast<int>(nb),
+                     count, loss);
+  SP_HIP(hipGetLastError());
+}
+
+void Network::run_backward(int batch) {
+  if (tiles_)
+    tile_backward(tiles_->shape, off_, param_, grad_, tiles_->buf, spec_, prm_, dout_, batch, stream_);
+  else
+    general_backward(batch);
 }
 
 Network::~Network() {
@@ -621,9 +751,11 @@ Network::~Network() {
 void Network::set_parameters(const float* host) {
   SP_CHECK(host != nullptr, "parameters needed");
   SP_HIP(hipMemcpyAsync(param_, host, off_.total * sizeof(float), hipMemcpyHostToDevice, stream_));
-  hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks(off_.total, 256)), dim3(256), 0, stream_, param_,
-                     param16_, off_.total);
+  if (param16_)
+    hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks(off_.total, 256)), dim3(256), 0, stream_, param_,
+                       param16_, off_.total);
   SP_HIP(hipGetLastError());
+  parameters_changed();
   SP_HIP(hipStreamSynchronize(stream_));
 }
 
@@ -651,7 +783,7 @@ void Network::upload_batch(const float* spectra, const float* params, const floa
     SP_HIP(hipMemcpyAsync(tgt_, target, batch * n * sizeof(float), hipMemcpyHostToDevice, stream_));
 }
 
-void Network::run_forward(int B) {
+void Network::general_forward(int B) {
   const int n = s_.n, M = s_.modes, W = s_.width, H = s_.hidden;
   hipLaunchKernelGGL(lift_forward, dim3(blocks(n, 256), W, B), dim3(256), 0, stream_, spec_, prm_,
                      param_ + off_.lift_w, param_ + off_.lift_b, v16_[0], W, n, s_.n_params);
@@ -690,7 +822,7 @@ void Network::run_forward(int B) {
   SP_HIP(hipGetLastError());
 }
 
-void Network::run_backward(int B) {
+void Network::general_backward(int B) {
   const int n = s_.n, M = s_.modes, W = s_.width, H = s_.hidden;
   const long Wn = static_cast<long>(W) * n;
   // Head.
@@ -745,7 +877,7 @@ void Network::run_backward(int B) {
 void Network::forward(const float* spectra, const float* params, int batch, float* out) {
   SP_CHECK(out != nullptr, "an output is needed");
   upload_batch(spectra, params, nullptr, batch);
-  run_forward(batch);
+  run_forward(batch, nullptr);
   SP_HIP(hipMemcpyAsync(out, out_, static_cast<long>(batch) * s_.n * sizeof(float),
                         hipMemcpyDeviceToHost, stream_));
   SP_HIP(hipStreamSynchronize(stream_));
@@ -755,16 +887,11 @@ double Network::gradient(const float* spectra, const float* params, const float*
                          int batch, float* grad) {
   SP_CHECK(target && grad, "a target and a gradient output are needed");
   upload_batch(spectra, params, target, batch);
-  run_forward(batch);
-  const long count = static_cast<long>(batch) * s_.n;
-  const unsigned nb = blocks(count, 256);
-  hipLaunchKernelGGL(loss_grad, dim3(nb), dim3(256), 0, stream_, out_, tgt_, dout_, partials_, count);
-  hipLaunchKernelGGL(loss_total, dim3(1), dim3(256), 0, stream_, partials_, static_cast<int>(nb),
-                     count, partials_ + nb);
-  SP_HIP(hipGetLastError());
+  float* sum = partials_ + blocks(static_cast<long>(batch) * s_.n, 256);
+  run_forward(batch, sum);
   run_backward(batch);
   float loss = 0.f;
-  SP_HIP(hipMemcpyAsync(&loss, partials_ + nb, sizeof(float), hipMemcpyDeviceToHost, stream_));
+  SP_HIP(hipMemcpyAsync(&loss, sum, sizeof(float), hipMemcpyDeviceToHost, stream_));
   SP_HIP(hipMemcpyAsync(grad, grad_, off_.total * sizeof(float), hipMemcpyDeviceToHost, stream_));
   SP_HIP(hipStreamSynchronize(stream_));
   return loss;
@@ -808,8 +935,6 @@ void Network::train(const int* indices, long steps, int batch, float lr, float* 
   }
   SP_HIP(hipMemcpyAsync(indices_, indices, steps * batch * sizeof(int), hipMemcpyHostToDevice,
                         stream_));
-  const long count = static_cast<long>(batch) * s_.n;
-  const unsigned nb = blocks(count, 256);
   const auto t0 = std::chrono::steady_clock::now();
   const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
   for (long step = 0; step < steps; ++step) {
@@ -817,12 +942,7 @@ void Network::train(const int* indices, long steps, int batch, float lr, float* 
                        indices_ + step * batch, ds_spec_, ds_prm_, ds_tgt_, spec_, prm_, tgt_, s_.n,
                        s_.n_params);
     SP_HIP(hipGetLastError());
-    run_forward(batch);
-    hipLaunchKernelGGL(loss_grad, dim3(nb), dim3(256), 0, stream_, out_, tgt_, dout_, partials_,
-                       count);
-    hipLaunchKernelGGL(loss_total, dim3(1), dim3(256), 0, stream_, partials_, static_cast<int>(nb),
-                       count, losses_ + step);
-    SP_HIP(hipGetLastError());
+    run_forward(batch, losses_ + step);
     run_backward(batch);
     adam_t_ += 1;
     const double c1 = 1.0 - std::pow(0.9, static_cast<double>(adam_t_));
@@ -831,6 +951,7 @@ void Network::train(const int* indices, long steps, int batch, float lr, float* 
     hipLaunchKernelGGL(adam, dim3(blocks(off_.total, 256)), dim3(256), 0, stream_, param_, param16_,
                        grad_, m_, v_, off_.total, step_size, beta1, beta2, eps);
     SP_HIP(hipGetLastError());
+    parameters_changed();
   }
   SP_HIP(hipMemcpyAsync(losses, losses_, steps * sizeof(float), hipMemcpyDeviceToHost, stream_));
   SP_HIP(hipStreamSynchronize(stream_));

@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -45,6 +46,8 @@ struct Offsets {
 };
 Offsets offsets(const Shape& s);
 
+struct TilePath;
+
 class Network {
  public:
   Network(const Shape& s, int max_batch);
@@ -70,9 +73,15 @@ class Network {
 
  private:
   void upload_batch(const float* spectra, const float* params, const float* target, int batch);
-  void run_forward(int batch);
-  void run_backward(int batch);  // needs d_out_ set; fills grad_
-  void zero_grad();
+  // The output of the uploaded batch; with `loss` also its mean squared error against
+  // tgt_, dout_ and what run_backward (which fills grad_) needs.
+  void run_forward(int batch, float* loss);
+  void run_backward(int batch);
+  void general_forward(int batch);
+  void general_backward(int batch);
+  void allocate_general();
+  void allocate_tiles();
+  void parameters_changed();
   Shape s_;
   Offsets off_;
   int max_batch_;
@@ -104,6 +113,8 @@ class Network {
   long losses_cap_ = 0;
   int* indices_ = nullptr;
   long indices_cap_ = 0;
+  // The fused tile path of narrow networks (fno_tile.hpp); null on the general path.
+  std::unique_ptr<TilePath> tiles_;
   // Dataset.
   float *ds_spec_ = nullptr, *ds_prm_ = nullptr, *ds_tgt_ = nullptr;
   long ds_n_ = 0;

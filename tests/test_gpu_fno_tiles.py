@@ -1,0 +1,67 @@
+"""GPU: the surrogate's fused tile path at the edges of its padding, and the general
+products of wider networks, against the FP64 oracle (``oracle/fno.py``).
+
+Channels pad to 32 or 64, twice the modes to 64 or 128, bins to tiles of 64 and samples
+to runs of 16; a batch splits each sample's tiles over workgroups by its size. The shapes
+below sit on and beside each of these edges. BF16 operands (unit roundoff 2^-9) pass
+through two products a layer forward and three back, so a tensor's relative error is a
+few 2^-9 sqrt(layers): the bounds are those of the other surrogate tests, 2 % and a cosine
+of 0.9995, which one wrong row, column or sign in a small tensor breaks.
+"""
+
+import numpy as np
+import pytest
+
+from oracle import fno as oracle
+from solprop_amd import surrogate
+from test_gpu_fno import case, rel
+
+pytestmark = pytest.mark.gpu
+
+# (width, modes, layers, hidden, n, scan parameters, batch)
+EDGES = [
+    (1, 1, 1, 1, 4, 0, 1),
+    (16, 8, 2, 32, 63, 1, 5),
+    (31, 32, 2, 33, 64, 4, 17),
+    (33, 33, 3, 127, 65, 8, 2),
+    (48, 24, 4, 64, 500, 4, 16),
+    (64, 64, 2, 128, 129, 4, 33),
+    (64, 64, 4, 128, 2048, 4, 3),
+    (64, 65, 2, 128, 256, 4, 3),
+    (65, 16, 2, 64, 256, 4, 3),
+    (32, 16, 2, 129, 256, 4, 3),
+]
+
+
+@pytest.mark.parametrize("edge", EDGES, ids=lambda e: "-".join(map(str, e)))
+def test_forward_and_gradient_at_the_edges(edge):
+    width, modes, layers, hidden, n, n_params, batch = edge
+    print("fno tiles", edge, flush=True)
+    shape = surrogate.Shape(n_params=n_params, width=width, modes=modes, layers=layers,
+                            hidden=hidden, n=n)
+    o, flat, spectra, params, target = case(shape, batch, seed=3)
+    net = surrogate.Network(shape, max_batch=batch + 3)
+    net.set_parameters(flat)
+    # A full batch first, so that a smaller one after it must not see its rows.
+    full = np.resize(spectra, (batch + 3, n)), np.resize(params, (batch + 3, n_params))
+    first = net.forward(*full)
+    got = net.forward(spectra, params)
+    loss, grad = net.gradient(spectra, params, target)
+    again = net.gradient(spectra, params, target)
+    net.close()
+    assert loss == again[0] and np.array_equal(grad, again[1])
+    x = surrogate.oracle_inputs(spectra, params)
+    loss_ref, grad_ref, out_ref = oracle.loss_and_grad(o, flat.astype(np.float64), x, target)
+    assert rel(got, out_ref) < 2e-2
+    assert rel(first[:batch], out_ref) < 2e-2
+    assert abs(loss - loss_ref) <= 2e-2 * loss_ref
+    at = 0
+    for name, shp in oracle.layout(o):
+        size = int(np.prod(shp))
+        g, r = grad[at:at + size].astype(np.float64), grad_ref[at:at + size]
+        at += size
+        norm = np.linalg.norm(r)
+        if norm < 1e-9 * np.linalg.norm(grad_ref):
+            continue  # a mode that the grid does not carry (the imaginary part at zero)
+        assert rel(g, r) < 2e-2, (name, rel(g, r))
+        assert g @ r / (np.linalg.norm(g) * norm) > 0.9995, name
