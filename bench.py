@@ -477,17 +477,18 @@ def run_fno(args):
 
 
 # Algorithmic bytes a launch moves, per point of the volume: a transform pass reads and
-# writes each complex point once (32); the t rows' forward pass also reads the prefactor
-# (48); the register passes read and write the low-storage registers (pass 1: y, source,
-# operator in, y, g, B, C out; 2: source, g, B, y in, B, C, g out; 3: source, g, B,
-# operator, y in, B, C out; 4: operator, B, source in, y out).
+# writes each complex point once (32); the t stages also read the prefactor and the
+# low-storage registers (stage 1: field, prefactor, operator, y in, y, g, field out;
+# 2: field, prefactor, g, y in, B, g, field out; 3: field, prefactor, g, B, operator, y in,
+# B, field out; 4: field, prefactor, operator, B in, y out), the prefactor and operator
+# their imaginary parts alone (the beam's medium is lossless).
 CARTESIAN_PHASE_BYTES = {
     "record upload": 0.0, "t inverse": 32.0, "x pass": 32.0, "y response": 32.0,
-    "t forward": 48.0, "ls pass 1": 112.0, "ls pass 2": 112.0, "ls pass 3": 112.0,
-    "ls pass 4": 64.0, "norms": 0.0,
+    "t stage 1": 96.0, "t stage 2": 104.0, "t stage 3": 112.0, "t stage 4": 64.0,
+    "norms": 0.0,
 }
-CARTESIAN_LAUNCHES = {"t inverse": 4, "x pass": 8, "y response": 4, "t forward": 4,
-                      "ls pass 1": 1, "ls pass 2": 1, "ls pass 3": 1, "ls pass 4": 1}
+CARTESIAN_LAUNCHES = {"t inverse": 1, "x pass": 8, "y response": 4, "t stage 1": 1,
+                      "t stage 2": 1, "t stage 3": 1, "t stage 4": 1}
 
 
 def run_cartesian(args):

@@ -8,7 +8,7 @@
 #include <functional>
 #include <string>
 
-#include "fft_lds.hpp"
+#include "fft_regs.hpp"
 #include "sync.hpp"
 
 namespace sp {
@@ -24,93 +24,249 @@ __device__ inline cplx kerr_point(cplx e, const KerrArgs& k) {
   return scale(k.coefficient, p);
 }
 
+// Every pass is bound by HBM: a volume does not fit the caches, so the passes' count of
+// volume reads and writes sets the time, and each pass has to keep enough of them in
+// flight. The transforms therefore run radix-16 stages in registers (fft_regs.hpp): a
+// thread's 16 loads are issued together, and a 256-point sequence crosses LDS once.
+// 256 x 128 x 512 points (268 MB a pass either way), before with radix-4 stages in LDS and
+// now: x pass 158 -> 84 us (6.4 TB/s), y response 140 -> 98 us.
+
+// The x axis: G neighbouring sequences (points `stride` apart, blocks of L stride points).
+template <int LOG2L, int G, int Sign>
+__global__ void __launch_bounds__((RegsFft<LOG2L, G, true, false>::NT))
+    cart_x(cplx* f, long stride, const cplx* __restrict__ tw) {
+  using F = RegsFft<LOG2L, G, true, false>;
+  __shared__ cplx lds[F::LDS_POINTS];
+  cplx* at = f + static_cast<long>(blockIdx.y) * F::L * stride + static_cast<long>(blockIdx.x) * G;
+  typename F::First v;
+  typename F::Last w;
+  F::inputs(v, [&](cplx& x, int s, int j) { x = at[j * stride + s]; });
+  F::run(v, w, lds, tw, Sign);
+  F::outputs(w, [&](cplx& x, int s, int j) { at[j * stride + s] = x; });
+}
+
 // The y axis's inverse transform, the response at every point and the forward transform
-// in one pass: G neighbouring y-sequences (points `stride` apart) staged in LDS, in place.
-// Each workgroup reads and writes only its own sequences.
+// in one pass, in place: the forward transform's stages run in the reverse order of
+// radices, so that it starts from the registers the inverse ends with.
 template <int LOG2L, int G>
-__global__ void __launch_bounds__((Shape<LOG2L, G>::NT))
+__global__ void __launch_bounds__((RegsFft<LOG2L, G, true, false>::NT))
     cart_y_response(cplx* f, long stride, const cplx* __restrict__ tw, KerrArgs k) {
-  using S = Shape<LOG2L, G>;
-  constexpr int E = S::E, NT = S::NT, STRIDE = S::STRIDE;
-  __shared__ cplx buf[G * STRIDE];
-  const long s0 = static_cast<long>(blockIdx.x) * G;
-  for (int e = threadIdx.x; e < E; e += NT) {
-    const int s = e % G, j = e / G;
-    buf[s * STRIDE + j] = f[j * stride + s0 + s];
-  }
-  __syncthreads();
-  lds_transform<LOG2L, G>(buf, tw, +1);
-  for (int e = threadIdx.x; e < E; e += NT) {
-    const int s = e % G, j = e / G;
-    buf[s * STRIDE + j] = kerr_point(buf[s * STRIDE + j], k);
-  }
-  __syncthreads();
-  lds_transform<LOG2L, G>(buf, tw, -1);
-  for (int e = threadIdx.x; e < E; e += NT) {
-    const int s = e % G, j = e / G;
-    f[j * stride + s0 + s] = buf[s * STRIDE + j];
+  using I = RegsFft<LOG2L, G, true, false>;
+  using F = RegsFft<LOG2L, G, true, true>;
+  __shared__ cplx lds[I::LDS_POINTS];
+  cplx* at = f + static_cast<long>(blockIdx.x) * G;
+  typename I::First v;
+  typename I::Last w;
+  I::inputs(v, [&](cplx& x, int s, int j) { x = at[j * stride + s]; });
+  I::run(v, w, lds, tw, +1);
+  // Both transforms order a butterfly's points alike; the inverse leaves them permuted.
+  typename F::First u;
+  constexpr int R = F::radix(0);
+#pragma unroll
+  for (int r = 0; r < F::template per<R>(); ++r)
+#pragma unroll
+    for (int j = 0; j < R; ++j) u[r][j] = kerr_point(w[r][out_at<R>(j)], k);
+  __syncthreads();  // the inverse's last hand-over is read
+  typename F::Last z;
+  F::run(u, z, lds, tw, -1);
+  F::outputs(z, [&](cplx& x, int s, int j) { at[j * stride + s] = x; });
+}
+
+// The t axis (contiguous rows) and what happens to its spectrum between two source
+// evaluations, so that the spectrum of a source and of the next stage's input are never
+// stored: G rows of the field are transformed forward in registers, laid out in LDS, and
+// a loop over the points applies the prefactor and the register pass of the low-storage
+// step (J. Hult, J. Lightwave Technol. 25, 3770 (2007), in the reference's three-register
+// form, src/solprop/backends/numpy_ref/engines.py:432-480): y the state A, acc the
+// accumulator, prev the previous source (for the stiffness indicator). R[0].x_w and
+// R[1].x_w weigh the operator to the middle and to the end. The next stage's input is
+// transformed back in registers and stored as the field. The kinds:
+//   kInverse  the spectrum `y` into the field (a step's first input)
+//   kSource   the source alone into `acc`
+//   kPass 1..3 forward, register pass, inverse; kPass 4 forward, register pass (the state).
+// Passes 2 to 4 leave a masked sum per workgroup (|S2 - g|^2, |S3 - S2|^2, |A|^2), in a
+// fixed order. On 256 x 128 x 512 points stages 1 to 4 take 325, 320, 376 and 242 us
+// (4.4 to 5.4 TB/s), a step 2.44 ms (5.95 with the transforms and the passes apart and
+// radix-4). A step moves 53 volumes, or 49.5 where the
+// tables are imaginary (69 with the transforms and the passes apart).
+enum TKind : int { kInverse = 0, kPass1, kPass2, kPass3, kPass4, kSource };
+
+struct TArgs {
+  cplx* f;
+  cplx *y, *acc, *prev;
+  const void* pref;  // a table of cplx, or with Imaginary of doubles (the imaginary parts)
+  const void* phi;
+  const unsigned char* scored;
+  const AdamsRecord* R;
+  double* sums;
+};
+
+// Imaginary: the operator and the prefactor have no real part (a lossless medium), and
+// their tables hold the imaginary part alone, half the bytes; the products are the same.
+template <bool Imaginary>
+__device__ inline cplx table_times(const void* table, long idx, cplx v) {
+  if constexpr (Imaginary) {
+    const double b = static_cast<const double*>(table)[idx];
+    return make(-(b * v.y), b * v.x);
+  } else {
+    return mul(static_cast<const cplx*>(table)[idx], v);
   }
 }
 
-// The t axis (contiguous rows of L): the inverse transform of G rows of the spectrum into
-// the field, and the forward transform of G rows of the field times the prefactor into
-// the source.
-template <int LOG2L, int G>
-__global__ void __launch_bounds__((Shape<LOG2L, G>::NT))
-    cart_t_inverse(const cplx* __restrict__ spectrum, cplx* __restrict__ f,
-                   const cplx* __restrict__ tw) {
-  using S = Shape<LOG2L, G>;
-  constexpr int L = S::L, E = S::E, NT = S::NT, STRIDE = S::STRIDE;
-  __shared__ cplx buf[G * STRIDE];
+template <bool Imaginary>
+__device__ inline cplx table_flow(const void* table, long idx, double w) {
+  if constexpr (Imaginary) {
+    double sine, cosine;
+    sincos(w * static_cast<const double*>(table)[idx], &sine, &cosine);
+    return make(cosine, sine);
+  } else {
+    return cexp(scale(w, static_cast<const cplx*>(table)[idx]));
+  }
+}
+
+template <int LOG2L, int G, int Kind, bool Imaginary>
+__global__ void __launch_bounds__((RegsFft<LOG2L, G, false, false>::NT))
+    cart_t(TArgs a, const cplx* __restrict__ tw) {
+  using F = RegsFft<LOG2L, G, false, false>;
+  constexpr int L = F::L, E = F::E, NT = F::NT;
+  __shared__ cplx lds[F::LDS_POINTS];
+  __shared__ double tree[NT];
   const long base = static_cast<long>(blockIdx.x) * E;
-  for (int e = threadIdx.x; e < E; e += NT) buf[(e / L) * STRIDE + e % L] = spectrum[base + e];
-  __syncthreads();
-  lds_transform<LOG2L, G>(buf, tw, +1);
-  for (int e = threadIdx.x; e < E; e += NT) f[base + e] = buf[(e / L) * STRIDE + e % L];
+  const int tid = threadIdx.x;
+  if constexpr (Kind != kInverse) {
+    typename F::First v;
+    typename F::Last w;
+    F::inputs(v, [&](cplx& x, int s, int j) { x = a.f[base + s * L + j]; });
+    F::run(v, w, lds, tw, -1);
+    __syncthreads();  // the last hand-over is read
+    F::outputs(w, [&](cplx& x, int s, int j) { lds[F::slot(s, j)] = x; });
+    __syncthreads();
+    double sq = 0.0;
+    const double h = a.R[0].dz;
+    const double flow_w = a.R[Kind == kPass1 ? 0 : 1].x_w[0];
+#pragma unroll 2
+    for (int e = tid; e < E; e += NT) {
+      const long idx = base + e;
+      cplx& slot = lds[F::slot(e / L, e % L)];
+      const cplx s = table_times<Imaginary>(a.pref, idx, slot);
+      const bool scored = Kind != kSource && a.scored[e % L] != 0;
+      if constexpr (Kind == kSource) {
+        a.acc[idx] = s;
+      } else if constexpr (Kind == kPass1) {
+        const cplx flow = table_flow<Imaginary>(a.phi, idx, flow_w);
+        const cplx state = mul(flow, a.y[idx]);
+        const cplx g = mul(flow, s);
+        a.y[idx] = state;
+        a.prev[idx] = g;
+        slot = add(state, scale(0.5 * h, g));
+      } else if constexpr (Kind == kPass2) {
+        const cplx g = a.prev[idx], state = a.y[idx];
+        const cplx d = sub(s, g);
+        if (scored) sq += norm2(d);
+        a.acc[idx] = add(add(state, scale(h / 6.0, g)), scale(h / 3.0, s));
+        a.prev[idx] = s;
+        slot = add(state, scale(0.5 * h, s));
+      } else if constexpr (Kind == kPass3) {
+        const cplx d = sub(s, a.prev[idx]);
+        if (scored) sq += norm2(d);
+        a.acc[idx] = add(a.acc[idx], scale(h / 3.0, s));
+        const cplx flow = table_flow<Imaginary>(a.phi, idx, flow_w);
+        slot = mul(flow, add(a.y[idx], scale(h, s)));
+      } else {
+        const cplx flow = table_flow<Imaginary>(a.phi, idx, flow_w);
+        const cplx state = add(mul(flow, a.acc[idx]), scale(h / 6.0, s));
+        a.y[idx] = state;
+        if (scored) sq += norm2(state);
+      }
+    }
+    if constexpr (Kind >= kPass2 && Kind <= kPass4) {
+      tree[tid] = sq;
+      __syncthreads();
+      for (int half = NT / 2; half > 0; half /= 2) {
+        if (tid < half) tree[tid] = tree[tid] + tree[tid + half];
+        __syncthreads();
+      }
+      if (tid == 0) a.sums[static_cast<long>(Kind - kPass2) * gridDim.x + blockIdx.x] = tree[0];
+    }
+  }
+  if constexpr (Kind <= kPass3) {
+    typename F::First v;
+    typename F::Last w;
+    if constexpr (Kind == kInverse) {
+      F::inputs(v, [&](cplx& x, int s, int j) { x = a.y[base + s * L + j]; });
+    } else {
+      __syncthreads();
+      F::inputs(v, [&](cplx& x, int s, int j) { x = lds[F::slot(s, j)]; });
+      __syncthreads();
+    }
+    F::run(v, w, lds, tw, +1);
+    F::outputs(w, [&](cplx& x, int s, int j) { a.f[base + s * L + j] = x; });
+  }
+}
+
+__global__ void find_real_part(const cplx* __restrict__ table, std::size_t n, int* found) {
+  bool any = false;
+  for (std::size_t i = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<std::size_t>(gridDim.x) * blockDim.x)
+    any = any || !(table[i].x == 0.0);
+  if (any) *found = 1;
+}
+
+__global__ void take_imaginary(const cplx* __restrict__ table, std::size_t n,
+                               double* __restrict__ out) {
+  for (std::size_t i = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<std::size_t>(gridDim.x) * blockDim.x)
+    out[i] = table[i].y;
 }
 
 template <int LOG2L, int G>
-__global__ void __launch_bounds__((Shape<LOG2L, G>::NT))
-    cart_t_forward(const cplx* __restrict__ f, const cplx* __restrict__ pref,
-                   cplx* __restrict__ out, const cplx* __restrict__ tw) {
-  using S = Shape<LOG2L, G>;
-  constexpr int L = S::L, E = S::E, NT = S::NT, STRIDE = S::STRIDE;
-  __shared__ cplx buf[G * STRIDE];
-  const long base = static_cast<long>(blockIdx.x) * E;
-  for (int e = threadIdx.x; e < E; e += NT) buf[(e / L) * STRIDE + e % L] = f[base + e];
-  __syncthreads();
-  lds_transform<LOG2L, G>(buf, tw, -1);
-  for (int e = threadIdx.x; e < E; e += NT)
-    out[base + e] = mul(pref[base + e], buf[(e / L) * STRIDE + e % L]);
-}
+struct XPass {
+  static void launch(dim3 grid, hipStream_t s, cplx* f, long stride, const cplx* tw, int sign) {
+    constexpr int NT = RegsFft<LOG2L, G, true, false>::NT;
+    if (sign > 0)
+      hipLaunchKernelGGL((cart_x<LOG2L, G, 1>), grid, dim3(NT), 0, s, f, stride, tw);
+    else
+      hipLaunchKernelGGL((cart_x<LOG2L, G, -1>), grid, dim3(NT), 0, s, f, stride, tw);
+  }
+};
 
 template <int LOG2L, int G>
 struct YResponse {
   static void launch(unsigned blocks, hipStream_t s, cplx* f, long stride, const cplx* tw,
                      KerrArgs k) {
-    hipLaunchKernelGGL((cart_y_response<LOG2L, G>), dim3(blocks), dim3(Shape<LOG2L, G>::NT), 0,
-                       s, f, stride, tw, k);
+    hipLaunchKernelGGL((cart_y_response<LOG2L, G>), dim3(blocks),
+                       dim3(RegsFft<LOG2L, G, true, false>::NT), 0, s, f, stride, tw, k);
   }
 };
 
 template <int LOG2L, int G>
-struct TInverse {
-  static void launch(unsigned blocks, hipStream_t s, const cplx* spectrum, cplx* f,
-                     const cplx* tw) {
-    hipLaunchKernelGGL((cart_t_inverse<LOG2L, G>), dim3(blocks), dim3(Shape<LOG2L, G>::NT), 0,
-                       s, spectrum, f, tw);
+struct TStage {
+  template <bool Imaginary>
+  static void launch(int kind, unsigned blocks, hipStream_t s, const TArgs& a, const cplx* tw) {
+    const dim3 grid(blocks), block(RegsFft<LOG2L, G, false, false>::NT);
+    switch (kind) {
+      case kInverse:  // reads neither table
+        hipLaunchKernelGGL((cart_t<LOG2L, G, kInverse, true>), grid, block, 0, s, a, tw);
+        break;
+      case kPass1:
+        hipLaunchKernelGGL((cart_t<LOG2L, G, kPass1, Imaginary>), grid, block, 0, s, a, tw);
+        break;
+      case kPass2:
+        hipLaunchKernelGGL((cart_t<LOG2L, G, kPass2, Imaginary>), grid, block, 0, s, a, tw);
+        break;
+      case kPass3:
+        hipLaunchKernelGGL((cart_t<LOG2L, G, kPass3, Imaginary>), grid, block, 0, s, a, tw);
+        break;
+      case kPass4:
+        hipLaunchKernelGGL((cart_t<LOG2L, G, kPass4, Imaginary>), grid, block, 0, s, a, tw);
+        break;
+      default:
+        hipLaunchKernelGGL((cart_t<LOG2L, G, kSource, Imaginary>), grid, block, 0, s, a, tw);
+    }
   }
 };
 
-template <int LOG2L, int G>
-struct TForward {
-  static void launch(unsigned blocks, hipStream_t s, const cplx* f, const cplx* pref, cplx* out,
-                     const cplx* tw) {
-    hipLaunchKernelGGL((cart_t_forward<LOG2L, G>), dim3(blocks), dim3(Shape<LOG2L, G>::NT), 0,
-                       s, f, pref, out, tw);
-  }
-};
-
+// The strided passes' shapes: workgroups of at most kMaxElems points.
 template <template <int, int> class Op, int LOG2L, typename... A>
 void dispatch_g(int log2g, A... a) {
   constexpr int L = 1 << LOG2L;
@@ -144,31 +300,68 @@ void dispatch(int log2l, int log2g, A... a) {
   SP_HIP(hipGetLastError());
 }
 
+// The t rows a workgroup owns (log2): enough for 2^10 points (one wave, so that its
+// barriers wait for nobody: stage 1 344 -> 325 us and stage 4 265 -> 242 us against 2^11
+// points on 512-point rows), or 2^8 where that would leave fewer than 256 workgroups; at
+// most 16 rows, which divide any grid's nx ny.
+constexpr int t_log2g(int log2l, bool wide) {
+  const int g = (wide ? 10 : 8) - log2l;
+  return g < 0 ? 0 : (g > 4 ? 4 : g);
+}
+
+template <int LOG2L>
+void dispatch_t_wide(bool wide, bool imaginary, int kind, long rows, hipStream_t s,
+                     const TArgs& a, const cplx* tw) {
+  constexpr int W = t_log2g(LOG2L, true), N = t_log2g(LOG2L, false);
+  const unsigned blocks = static_cast<unsigned>(rows >> (wide ? W : N));
+  if (wide && imaginary)
+    TStage<LOG2L, (1 << W)>::template launch<true>(kind, blocks, s, a, tw);
+  else if (wide)
+    TStage<LOG2L, (1 << W)>::template launch<false>(kind, blocks, s, a, tw);
+  else if (imaginary)
+    TStage<LOG2L, (1 << N)>::template launch<true>(kind, blocks, s, a, tw);
+  else
+    TStage<LOG2L, (1 << N)>::template launch<false>(kind, blocks, s, a, tw);
+}
+
+void dispatch_t(int log2l, bool wide, bool imaginary, int kind, long rows, hipStream_t s,
+                const TArgs& a, const cplx* tw) {
+  switch (log2l) {
+    case 2: dispatch_t_wide<2>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 3: dispatch_t_wide<3>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 4: dispatch_t_wide<4>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 5: dispatch_t_wide<5>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 6: dispatch_t_wide<6>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 7: dispatch_t_wide<7>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 8: dispatch_t_wide<8>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 9: dispatch_t_wide<9>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 10: dispatch_t_wide<10>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 11: dispatch_t_wide<11>(wide, imaginary, kind, rows, s, a, tw); break;
+    case 12: dispatch_t_wide<12>(wide, imaginary, kind, rows, s, a, tw); break;
+    default: throw Error(kValue, "a Cartesian axis has 4 to 4096 points");
+  }
+  SP_HIP(hipGetLastError());
+}
+
 int log2_of(int n) {
   int m = 0;
   while ((1 << m) < n) ++m;
   return m;
 }
 
-// Sequences a workgroup owns on an axis of n points with `count` sequences: contiguous
-// runs of up to 16 points across the sequences (a strided axis), or for the contiguous t
-// rows enough rows for 256 points at least; never more than `max_points` points.
-int axis_log2g(int n, long count, bool strided, int max_points) {
+// Sequences a workgroup of a strided pass owns: runs of up to 16 neighbouring points,
+// never more than `max_points` points in all.
+int axis_log2g(int n, long count, int max_points) {
   int g = 0;
-  const long want = strided ? 16 : std::max(1, 256 / n);
   const int cap = std::min(max_points, kMaxElems);
-  while ((1L << (g + 1)) <= want && n * (1 << (g + 1)) <= cap && (1L << (g + 1)) <= count &&
-         count % (1L << (g + 1)) == 0)
-    ++g;
+  while (g < 4 && n * (1 << (g + 1)) <= cap && count % (1L << (g + 1)) == 0) ++g;
   return g;
 }
 
-enum Phase : int {
-  kUpload, kPassT, kPassX, kPassY, kFinish, kLs1, kLs2, kLs3, kLs4, kNorms
-};
+enum Phase : int { kUpload, kPassT, kPassX, kPassY, kLs1, kLs2, kLs3, kLs4, kNorms };
 const char* const kPhaseNames[] = {"record upload", "t inverse", "x pass", "y response",
-                                   "t forward", "ls pass 1", "ls pass 2", "ls pass 3",
-                                   "ls pass 4", "norms"};
+                                   "t stage 1", "t stage 2", "t stage 3", "t stage 4",
+                                   "norms"};
 
 struct ReplayEngine final : march::Engine {
   std::function<double(double, double)> step;
@@ -241,8 +434,11 @@ CartesianWorkspace::CartesianWorkspace(const sp_problem_desc& d) {
   SP_CHECK(max_points >= 4 && max_points <= 4096,
            "SOLPROP_MI355X_CARTESIAN_TILE is 4 to 4096 points");
   const long rows = static_cast<long>(nx_) * ny_;
-  gt_ = axis_log2g(nt_, rows, false, 4096);
-  gy_ = axis_log2g(ny_, static_cast<long>(nx_) * nt_, true, max_points);
+  const int lt = log2_of(nt_);
+  wide_t_ = (rows >> t_log2g(lt, true)) >= 256;
+  t_blocks_ = static_cast<int>(rows >> t_log2g(lt, wide_t_));
+  gx_ = axis_log2g(nx_, nt_, max_points);
+  gy_ = axis_log2g(ny_, static_cast<long>(nx_) * nt_, max_points);
   try {
     SP_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     const int C = nx_ * ny_, N = nt_;
@@ -261,30 +457,52 @@ CartesianWorkspace::CartesianWorkspace(const sp_problem_desc& d) {
     auto* nm = alloc<unsigned char>(N);
     SP_HIP(hipMemcpy(nm, d.norm_mask, N, hipMemcpyHostToDevice));
     P_.normmask = nm;
-    auto* phi = alloc<cplx>(V_);
-    SP_HIP(hipMemcpy(phi, d.phi_terms, V_ * sizeof(cplx), hipMemcpyHostToDevice));
-    P_.phi = phi;
-    auto* pref = alloc<cplx>(V_);
-    SP_HIP(hipMemcpy(pref, d.prefactor_terms, V_ * sizeof(cplx), hipMemcpyHostToDevice));
-    P_.pref = pref;
     B_.y = alloc<cplx>(V_);
-    B_.lab = alloc<cplx>(V_);
-    B_.source = alloc<cplx>(V_);
     B_.advanced = alloc<cplx>(V_);
     field_ = alloc<cplx>(V_);
     acc_ = alloc<cplx>(V_);
     prev_ = alloc<cplx>(V_);
     save_ = alloc<cplx>(V_);
-    plan_t_.init(static_cast<std::size_t>(nt_), static_cast<std::size_t>(nx_) * ny_);
-    // Columns iy nx + ix: the x axis has stride nt within each of ny blocks, the y axis
-    // stride nx nt.
-    plan_x_.init_axis(static_cast<std::size_t>(nx_), static_cast<std::size_t>(nt_),
-                      static_cast<std::size_t>(ny_), static_cast<std::size_t>(max_points));
-    plan_y_.init_axis(static_cast<std::size_t>(ny_), static_cast<std::size_t>(nx_) * nt_, 1);
+    // The tables' layout is decided, and the imaginary parts taken, on the device.
+    auto* real_part = alloc<int>(1);
+    SP_HIP(hipMemcpy(save_, d.phi_terms, V_ * sizeof(cplx), hipMemcpyHostToDevice));
+    SP_HIP(hipMemcpy(field_, d.prefactor_terms, V_ * sizeof(cplx), hipMemcpyHostToDevice));
+    SP_HIP(hipMemsetAsync(real_part, 0, sizeof(int), stream_));
+    const dim3 grid(4096), block(256);
+    hipLaunchKernelGGL(find_real_part, grid, block, 0, stream_, save_, V_, real_part);
+    hipLaunchKernelGGL(find_real_part, grid, block, 0, stream_, field_, V_, real_part);
+    SP_HIP(hipGetLastError());
+    int found = 0;
+    SP_HIP(hipStreamSynchronize(stream_));
+    SP_HIP(hipMemcpy(&found, real_part, sizeof(int), hipMemcpyDeviceToHost));
+    imaginary_ = found == 0;
+    auto table = [&](const cplx* src) -> const void* {
+      if (imaginary_) {
+        auto* p = alloc<double>(V_);
+        hipLaunchKernelGGL(take_imaginary, grid, block, 0, stream_, src, V_, p);
+        SP_HIP(hipGetLastError());
+        return p;
+      }
+      auto* p = alloc<cplx>(V_);
+      SP_HIP(hipMemcpyAsync(p, src, V_ * sizeof(cplx), hipMemcpyDeviceToDevice, stream_));
+      return p;
+    };
+    phi_ = table(save_);
+    pref_ = table(field_);
+    SP_HIP(hipStreamSynchronize(stream_));
+    auto roots = [&](int n) {
+      const auto host = unit_roots(static_cast<std::size_t>(n));
+      auto* p = alloc<cplx>(host.size());
+      SP_HIP(hipMemcpy(p, host.data(), host.size() * sizeof(cplx), hipMemcpyHostToDevice));
+      return p;
+    };
+    roots_t_ = roots(nt_);
+    roots_x_ = roots(nx_);
+    roots_y_ = roots(ny_);
     rec_dev_ = alloc<AdamsRecord>(3);
     SP_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec_host_), 3 * sizeof(AdamsRecord)));
     std::memset(rec_host_, 0, 3 * sizeof(AdamsRecord));
-    partials_ = alloc<double>(ls_partials(P_));
+    partials_ = alloc<double>(ls_partials(static_cast<unsigned>(t_blocks_)));
     SP_HIP(hipHostMalloc(reinterpret_cast<void**>(&norms_host_), 4 * sizeof(double),
                          hipHostMallocMapped));
     SP_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&B_.norms), norms_host_, 0));
@@ -347,28 +565,30 @@ std::vector<std::pair<const char*, double>> CartesianWorkspace::phases() const {
   return out;
 }
 
-void CartesianWorkspace::enqueue_source(const cplx* spectrum) {
-  // E = FFT3^-1[Y] over t, x, then y; the response between the y axis's inverse and
-  // forward transforms in one pass; then forward over x and t, the prefactor applied as
-  // the t rows are stored.
-  const long rows = static_cast<long>(nx_) * ny_;
-  const int lt = log2_of(nt_), ly = log2_of(ny_);
-  const int gt = gt_, gy = gy_;
+void CartesianWorkspace::enqueue_t(int kind, int phase) {
+  const TArgs a{field_, B_.y, acc_, prev_, pref_, phi_, P_.normmask, rec_dev_, partials_};
+  dispatch_t(log2_of(nt_), wide_t_, imaginary_, kind, static_cast<long>(nx_) * ny_, stream_, a, roots_t_);
+  mark(phase);
+}
+
+// The transverse axes of a source evaluation, on the field the t rows' inverse left:
+// x, then y with the response between its inverse and forward transforms, then x.
+// Columns are iy nx + ix: the x axis has stride nt within each of ny blocks, the y axis
+// stride nx nt.
+void CartesianWorkspace::enqueue_transverse() {
   const long y_seqs = static_cast<long>(nx_) * nt_;
   const KerrArgs k{kerr_scale_, kerr_self_, kerr_conj_};
-  dispatch<TInverse>(lt, gt, static_cast<unsigned>(rows >> gt), stream_, spectrum, field_,
-                     plan_t_.roots());
-  mark(kPassT);
-  plan_x_.exec(field_, nullptr, +1, stream_);
+  const dim3 x_grid(static_cast<unsigned>(nt_ >> gx_), static_cast<unsigned>(ny_));
+  const int lx = log2_of(nx_);
+  dispatch<XPass>(lx, gx_, x_grid, stream_, field_, static_cast<long>(nt_),
+                  static_cast<const cplx*>(roots_x_), +1);
   mark(kPassX);
-  dispatch<YResponse>(ly, gy, static_cast<unsigned>(y_seqs >> gy), stream_, field_, y_seqs,
-                      plan_y_.roots(), k);
+  dispatch<YResponse>(log2_of(ny_), gy_, static_cast<unsigned>(y_seqs >> gy_), stream_, field_,
+                      y_seqs, static_cast<const cplx*>(roots_y_), k);
   mark(kPassY);
-  plan_x_.exec(field_, nullptr, -1, stream_);
+  dispatch<XPass>(lx, gx_, x_grid, stream_, field_, static_cast<long>(nt_),
+                  static_cast<const cplx*>(roots_x_), -1);
   mark(kPassX);
-  dispatch<TForward>(lt, gt, static_cast<unsigned>(rows >> gt), stream_,
-                     static_cast<const cplx*>(field_), P_.pref, B_.source, plan_t_.roots());
-  mark(kFinish);
 }
 
 void CartesianWorkspace::enqueue_step() {
@@ -376,19 +596,12 @@ void CartesianWorkspace::enqueue_step() {
   SP_HIP(hipMemcpyAsync(rec_dev_, rec_host_, 3 * sizeof(AdamsRecord), hipMemcpyHostToDevice,
                         stream_));
   mark(kUpload);
-  enqueue_source(B_.y);
-  launch_ls_pass(1, P_, rec_dev_, B_, acc_, prev_, partials_, stream_);
-  mark(kLs1);
-  enqueue_source(B_.lab);
-  launch_ls_pass(2, P_, rec_dev_, B_, acc_, prev_, partials_, stream_);
-  mark(kLs2);
-  enqueue_source(B_.lab);
-  launch_ls_pass(3, P_, rec_dev_, B_, acc_, prev_, partials_, stream_);
-  mark(kLs3);
-  enqueue_source(B_.lab);
-  launch_ls_pass(4, P_, rec_dev_, B_, acc_, prev_, partials_, stream_);
-  mark(kLs4);
-  launch_ls_norms(P_, partials_, B_.norms, stream_);
+  enqueue_t(kInverse, kPassT);
+  for (int pass = 0; pass < 4; ++pass) {
+    enqueue_transverse();
+    enqueue_t(kPass1 + pass, kLs1 + pass);
+  }
+  launch_ls_norms(static_cast<unsigned>(t_blocks_), partials_, B_.norms, stream_);
   mark(kNorms);
 }
 
@@ -450,7 +663,6 @@ void CartesianWorkspace::load(double z, const double* field) {
 double CartesianWorkspace::probe_trial(double z, double dz) {
   if (!loaded_) throw Error(kState, "load a state before taking a trial");
   SP_HIP(hipMemcpyAsync(save_, B_.y, V_ * sizeof(cplx), hipMemcpyDeviceToDevice, stream_));
-  // The transforms' scratch is `save_` only for a four-step time axis (nt > 4096, refused).
   const double norm = trial(z, dz);
   SP_HIP(hipMemcpyAsync(B_.advanced, B_.y, V_ * sizeof(cplx), hipMemcpyDeviceToDevice, stream_));
   SP_HIP(hipMemcpyAsync(B_.y, save_, V_ * sizeof(cplx), hipMemcpyDeviceToDevice, stream_));
@@ -530,8 +742,7 @@ sp_counters CartesianWorkspace::counters() const {
   c.evaluations = evaluations_;
   c.accepted = accepted_;
   c.graph_launches = graph_launches_;
-  c.device_bytes = static_cast<long>(device_bytes_ + plan_t_.bytes() + plan_y_.bytes() +
-                                     plan_x_.bytes());
+  c.device_bytes = static_cast<long>(device_bytes_);
   return c;
 }
 
@@ -553,10 +764,15 @@ void CartesianWorkspace::source(double z, const double* lab, double* out, double
   (void)z;
   SP_CHECK(lab && out && !streams && !modal, "the Cartesian source takes a spectrum and an output");
   SP_HIP(hipStreamSynchronize(stream_));
-  SP_HIP(hipMemcpy(B_.lab, lab, V_ * sizeof(cplx), hipMemcpyHostToDevice));
-  enqueue_source(B_.lab);
+  // The state is kept: the spectrum takes its place for the inverse transform only.
+  SP_HIP(hipMemcpy(save_, B_.y, V_ * sizeof(cplx), hipMemcpyDeviceToDevice));
+  SP_HIP(hipMemcpy(B_.y, lab, V_ * sizeof(cplx), hipMemcpyHostToDevice));
+  enqueue_t(kInverse, kPassT);
+  SP_HIP(hipMemcpyAsync(B_.y, save_, V_ * sizeof(cplx), hipMemcpyDeviceToDevice, stream_));
+  enqueue_transverse();
+  enqueue_t(kSource, kLs1);
   SP_HIP(hipStreamSynchronize(stream_));
-  SP_HIP(hipMemcpy(out, B_.source, V_ * sizeof(cplx), hipMemcpyDeviceToHost));
+  SP_HIP(hipMemcpy(out, acc_, V_ * sizeof(cplx), hipMemcpyDeviceToHost));
 }
 
 long CartesianWorkspace::buffer(const char* name, double* out, long count) {

@@ -10,12 +10,11 @@
 // operator is one constant table D(ky, kx, w) (the flows exp(D dz) formed per element),
 // its source S(Y) = p(ky, kx, w) FFT3[gamma |E|^2 E] with E = FFT3^-1[Y] / V, V = nx ny nt:
 // the analytic (envelope) Kerr response at every point of the volume, its conjugate term
-// for a response that keeps it. A source evaluation is five passes over the volume, each
-// a Stockham transform of whole axis sequences staged in LDS: the t rows' inverse from the
-// spectrum, the x axis's inverse, the y axis's inverse, response and forward in one pass,
-// the x axis's forward, the t rows' forward with the prefactor applied as they are stored
-// (the strided axes with a workgroup owning up to 16 neighbouring sequences, so that every
-// load and store moves contiguous runs).
+// for a response that keeps it. A source evaluation's transverse
+// axes are three passes over the volume (x inverse; y inverse, response and y forward; x
+// forward), a workgroup owning up to 16 neighbouring sequences so that every load and
+// store moves contiguous runs; the t rows' forward transform, the prefactor, the register
+// pass of the low-storage step and the next stage's inverse transform are one more.
 #pragma once
 
 #include <utility>
@@ -63,7 +62,8 @@ class CartesianWorkspace final : public Propagator {
   template <typename T>
   T* alloc(std::size_t n);
   void release();
-  void enqueue_source(const cplx* spectrum);  // into B_.source
+  void enqueue_t(int kind, int phase);  // a t-axis pass (cartesian.hip's kinds)
+  void enqueue_transverse();
   void enqueue_step();
   double trial(double z, double dz);
   void wait();
@@ -71,14 +71,18 @@ class CartesianWorkspace final : public Propagator {
   void collect();        // profiling: the marked launches' times into their phases
 
   int nx_ = 0, ny_ = 0, nt_ = 0;
-  int gt_ = 0, gy_ = 0;  // log2 of the sequences a workgroup owns: t rows, y axis
+  int gx_ = 0, gy_ = 0;  // log2 of the sequences a workgroup owns: x axis, y axis
+  bool imaginary_ = false;  // the operator and prefactor tables have no real part
+  const void *phi_ = nullptr, *pref_ = nullptr;
+  bool wide_t_ = true;   // the t rows' workgroups hold 2^11 points
+  int t_blocks_ = 0;
   std::size_t V_ = 0;
   DeviceProblem P_{};
   FieldBuffers B_{};
   std::vector<void*> allocations_;
   std::size_t device_bytes_ = 0;
   hipStream_t stream_ = nullptr;
-  FftPlan plan_t_, plan_y_, plan_x_;
+  cplx *roots_t_ = nullptr, *roots_x_ = nullptr, *roots_y_ = nullptr;  // unit roots
   cplx* field_ = nullptr;  // the (y, x, t) samples the transforms and the response act on
   cplx *acc_ = nullptr, *prev_ = nullptr, *save_ = nullptr;
   double kerr_self_ = 1.0, kerr_conj_ = 0.0, kerr_scale_ = 0.0;
@@ -94,8 +98,8 @@ class CartesianWorkspace final : public Propagator {
   bool loaded_ = false;
   double stiffness_ = 0.0;
   long trials_ = 0, evaluations_ = 0, accepted_ = 0, graph_launches_ = 0;
-  static constexpr int kPhases = 10;
-  static constexpr int kMarks = 64;  // events a profiled trial records (it needs 27)
+  static constexpr int kPhases = 9;
+  static constexpr int kMarks = 64;  // events a profiled trial records (it needs 19)
   bool profile_ = false, marking_ = false;
   std::vector<hipEvent_t> events_;
   std::vector<int> marked_;  // the phase each recorded event ends

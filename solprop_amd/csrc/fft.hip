@@ -514,46 +514,6 @@ void FftPlan::layout(std::size_t n, std::size_t batch) {
     SP_CHECK(kernel_for(p.log2L, p.log2G) != nullptr, "no FFT pass kernel for this shape");
 }
 
-void FftPlan::init_axis(std::size_t n, std::size_t inner, std::size_t outer,
-                        std::size_t max_points) {
-  SP_CHECK(n >= 4 && (n & (n - 1)) == 0 && n <= static_cast<std::size_t>(kMaxElems),
-           "an axis transform has a power-of-two length from 4 to 4096");
-  SP_CHECK(inner >= 1 && outer >= 1 && inner <= (std::size_t{1} << 30),
-           "an axis transform's strides must be positive");
-  n_ = n;
-  batch_ = outer;
-  owns_tables_ = true;
-  passes_.clear();
-  const int m = ilog2(n);
-  FftPass p;
-  p.log2L = m;
-  // Sequences a workgroup owns: as many neighbours as LDS holds (at most 16, 256 bytes
-  // of each row), so that every load and store moves contiguous runs of G points.
-  int g = 0;
-  const std::size_t cap = std::min(max_points, static_cast<std::size_t>(kMaxElems));
-  while (g < 4 && (std::size_t{1} << (m + g + 1)) <= cap && (std::size_t{1} << (g + 1)) <= inner &&
-         inner % (std::size_t{1} << (g + 1)) == 0)
-    ++g;
-  p.log2G = g;
-  p.in_sj = static_cast<long>(inner);
-  p.in_ss = 1;
-  p.out_sk = static_cast<long>(inner);
-  p.out_ss = 1;
-  // Rows are the outer blocks; a single block needs no row stride.
-  p.batch_in = p.batch_out = outer > 1 ? static_cast<long>(n * inner) : 0;
-  p.n_seq = static_cast<int>(inner);
-  passes_.push_back(p);
-  SP_CHECK(kernel_for(p.log2L, p.log2G) != nullptr, "no FFT pass kernel for this shape");
-  auto upload = [&](std::size_t len, cplx** dst) {
-    const auto host = unit_roots(len);
-    SP_HIP(hipMalloc(dst, len * sizeof(cplx)));
-    SP_HIP(hipMemcpy(*dst, host.data(), len * sizeof(cplx), hipMemcpyHostToDevice));
-    bytes_ += len * sizeof(cplx);
-  };
-  upload(n, &roots_n_);
-  upload(n, &roots_l_[0]);
-}
-
 std::size_t FftPlan::table_points(std::size_t n) {
   if (n <= static_cast<std::size_t>(kMaxElems)) return 2 * n;
   const int m = ilog2(n);

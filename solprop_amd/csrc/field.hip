@@ -1742,10 +1742,9 @@ __device__ inline cplx ls_flow(const DeviceProblem& P, const double* w, long idx
   return cexp(x);
 }
 
-// With Finish (the field route) a pass finishes its bin's source from the forward
-// transform's streams itself, at its evaluation's record (R[0] for pass 1, R[1] for passes
-// 2 and 3, R[2] for pass 4), instead of reading B.source.
-template <int Pass, bool Finish>
+// A pass finishes its bin's source from the forward transform's streams, at its
+// evaluation's record (R[0] for pass 1, R[1] for passes 2 and 3, R[2] for pass 4).
+template <int Pass>
 __global__ void __launch_bounds__(kLsThreads)
     ls_pass(DeviceProblem P, const AdamsRecord* __restrict__ R, FieldBuffers B, cplx* acc,
             cplx* prev, double* partials) {
@@ -1756,9 +1755,8 @@ __global__ void __launch_bounds__(kLsThreads)
   double sq = 0.0;
   if (idx < CN) {
     constexpr int at = Pass == 1 ? 0 : (Pass == 4 ? 2 : 1);
-    const cplx s = Finish ? finish_at(P, R[at], B, static_cast<int>(idx / P.N),
-                                      static_cast<int>(idx % P.N))
-                          : B.source[idx];
+    const cplx s = finish_at(P, R[at], B, static_cast<int>(idx / P.N),
+                             static_cast<int>(idx % P.N));
     const bool scored = P.normmask[idx % P.N] != 0;
     if constexpr (Pass == 1) {
       const cplx flow = ls_flow(P, R[0].x_w, idx, CN);
@@ -2353,38 +2351,25 @@ unsigned ls_blocks(const DeviceProblem& P) {
   return blocks_for(static_cast<std::size_t>(P.C) * P.N, kLsThreads);
 }
 
-std::size_t ls_partials(const DeviceProblem& P) {
-  const std::size_t blocks = ls_blocks(P);
-  const std::size_t runs = (blocks + kLsRun - 1) / kLsRun;
-  return 3 * blocks + (blocks > kLsRun ? 3 * runs : 0);
+std::size_t ls_partials(unsigned blocks) {
+  const std::size_t n = blocks, runs = (n + kLsRun - 1) / kLsRun;
+  return 3 * n + (n > kLsRun ? 3 * runs : 0);
 }
 
-namespace {
-template <bool Finish>
-void launch_ls_pass_for(int pass, const DeviceProblem& P, const AdamsRecord* R, FieldBuffers B,
-                        cplx* acc, cplx* prev, double* partials, hipStream_t s) {
+void launch_ls_pass(int pass, const DeviceProblem& P, const AdamsRecord* R, FieldBuffers B,
+                    cplx* acc, cplx* prev, double* partials, hipStream_t s) {
   const dim3 grid(ls_blocks(P)), block(kLsThreads);
   switch (pass) {
-    case 1: hipLaunchKernelGGL((ls_pass<1, Finish>), grid, block, 0, s, P, R, B, acc, prev, partials); break;
-    case 2: hipLaunchKernelGGL((ls_pass<2, Finish>), grid, block, 0, s, P, R, B, acc, prev, partials); break;
-    case 3: hipLaunchKernelGGL((ls_pass<3, Finish>), grid, block, 0, s, P, R, B, acc, prev, partials); break;
-    default: hipLaunchKernelGGL((ls_pass<4, Finish>), grid, block, 0, s, P, R, B, acc, prev, partials); break;
+    case 1: hipLaunchKernelGGL(ls_pass<1>, grid, block, 0, s, P, R, B, acc, prev, partials); break;
+    case 2: hipLaunchKernelGGL(ls_pass<2>, grid, block, 0, s, P, R, B, acc, prev, partials); break;
+    case 3: hipLaunchKernelGGL(ls_pass<3>, grid, block, 0, s, P, R, B, acc, prev, partials); break;
+    default: hipLaunchKernelGGL(ls_pass<4>, grid, block, 0, s, P, R, B, acc, prev, partials); break;
   }
   SP_HIP(hipGetLastError());
 }
-}  // namespace
 
-void launch_ls_pass(int pass, const DeviceProblem& P, const AdamsRecord* R, FieldBuffers B,
-                    cplx* acc, cplx* prev, double* partials, hipStream_t s, bool finish) {
-  if (finish)
-    launch_ls_pass_for<true>(pass, P, R, B, acc, prev, partials, s);
-  else
-    launch_ls_pass_for<false>(pass, P, R, B, acc, prev, partials, s);
-}
-
-void launch_ls_norms(const DeviceProblem& P, const double* partials, double* norms,
-                     hipStream_t s) {
-  const int blocks = static_cast<int>(ls_blocks(P));
+void launch_ls_norms(unsigned count, const double* partials, double* norms, hipStream_t s) {
+  const int blocks = static_cast<int>(count);
   if (blocks <= kLsRun) {
     hipLaunchKernelGGL(ls_norms, dim3(1), dim3(kLsThreads), 0, s, partials, blocks, norms);
   } else {

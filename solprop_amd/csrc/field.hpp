@@ -247,15 +247,13 @@ void launch_adams_norms(const DeviceProblem& P, FieldBuffers B, hipStream_t s);
 // The low-storage RK4IP step's register passes (1..4, each after its source evaluation)
 // and the three masked sums they leave (|S2 - g|^2, |S3 - S2|^2, |A|^2) into `norms`.
 unsigned ls_blocks(const DeviceProblem& P);
-// Doubles of the passes' partial sums: three rows of ls_blocks, and above kLsRun
+// Doubles of the passes' partial sums: three rows of `blocks`, and above kLsRun
 // workgroups three rows of the first level's run sums after them.
-std::size_t ls_partials(const DeviceProblem& P);
-// With `finish` (the field route) each pass finishes its bin's source from the forward
-// transform's streams instead of reading B.source.
+std::size_t ls_partials(unsigned blocks);
+// Each pass finishes its bin's source from the forward transform's streams.
 void launch_ls_pass(int pass, const DeviceProblem& P, const AdamsRecord* R, FieldBuffers B,
-                    cplx* acc, cplx* prev, double* partials, hipStream_t s,
-                    bool finish = false);
-void launch_ls_norms(const DeviceProblem& P, const double* partials, double* norms,
+                    cplx* acc, cplx* prev, double* partials, hipStream_t s);
+void launch_ls_norms(unsigned blocks, const double* partials, double* norms,
                      hipStream_t s);
 // Commits the held trial into store slot `slot`; reads no record, so the host may go on
 // filling the next trial's record while it runs.

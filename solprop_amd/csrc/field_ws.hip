@@ -275,7 +275,7 @@ void FieldWorkspace::allocate(const sp_problem_desc& d) {
     ls_rec_dev_ = alloc<AdamsRecord>(3);
     SP_HIP(hipHostMalloc(reinterpret_cast<void**>(&ls_rec_host_), 3 * sizeof(AdamsRecord)));
     std::memset(ls_rec_host_, 0, 3 * sizeof(AdamsRecord));
-    ls_partials_ = alloc<double>(ls_partials(P_));
+    ls_partials_ = alloc<double>(ls_partials(ls_blocks(P_)));
   }
   for (hipEvent_t& e : marks_) SP_HIP(hipEventCreate(&e));
   SP_HIP(hipEventCreateWithFlags(&done_, hipEventDisableTiming));
@@ -682,14 +682,14 @@ void FieldWorkspace::enqueue_ls_step() {
   // the midpoint; pass 4 at the end.
   // Each pass finishes its own bins' source (no finish launch between them).
   enqueue_source(B_.y, B_.source, ls_rec_dev_, false);
-  launch_ls_pass(1, P_, ls_rec_dev_, B_, ls_acc_, ls_prev_, ls_partials_, stream_, true);
+  launch_ls_pass(1, P_, ls_rec_dev_, B_, ls_acc_, ls_prev_, ls_partials_, stream_);
   enqueue_source(B_.lab, B_.source, ls_rec_dev_ + 1, false);
-  launch_ls_pass(2, P_, ls_rec_dev_, B_, ls_acc_, ls_prev_, ls_partials_, stream_, true);
+  launch_ls_pass(2, P_, ls_rec_dev_, B_, ls_acc_, ls_prev_, ls_partials_, stream_);
   enqueue_source(B_.lab, B_.source, ls_rec_dev_ + 1, false);
-  launch_ls_pass(3, P_, ls_rec_dev_, B_, ls_acc_, ls_prev_, ls_partials_, stream_, true);
+  launch_ls_pass(3, P_, ls_rec_dev_, B_, ls_acc_, ls_prev_, ls_partials_, stream_);
   enqueue_source(B_.lab, B_.source, ls_rec_dev_ + 2, false);
-  launch_ls_pass(4, P_, ls_rec_dev_, B_, ls_acc_, ls_prev_, ls_partials_, stream_, true);
-  launch_ls_norms(P_, ls_partials_, B_.norms, stream_);
+  launch_ls_pass(4, P_, ls_rec_dev_, B_, ls_acc_, ls_prev_, ls_partials_, stream_);
+  launch_ls_norms(ls_blocks(P_), ls_partials_, B_.norms, stream_);
 }
 
 double FieldWorkspace::ls_trial(double z, double dz) {
