@@ -652,8 +652,7 @@ void CartesianWorkspace::load(double z, const double* field) {
   for (std::size_t i = 0; i < edges_.size(); ++i)
     if (march::reached(z, edges_[i]) && march::reached(edges_[i], z)) cursor = static_cast<long>(i);
   SP_CHECK(cursor >= 0, "a replay loads its state at one of its schedule's edges");
-  SP_HIP(hipStreamSynchronize(stream_));
-  SP_HIP(hipMemcpy(B_.y, field, V_ * sizeof(cplx), hipMemcpyHostToDevice));
+  transfer_.upload(B_.y, field, V_ * sizeof(cplx), stream_);
   state_ = march::State{};
   state_.z = edges_[static_cast<std::size_t>(cursor)];
   state_.cursor = cursor;
@@ -671,14 +670,12 @@ double CartesianWorkspace::probe_trial(double z, double dz) {
 }
 
 void CartesianWorkspace::read_trial(double* out) {
-  SP_HIP(hipStreamSynchronize(stream_));
-  SP_HIP(hipMemcpy(out, B_.advanced, V_ * sizeof(cplx), hipMemcpyDeviceToHost));
+  transfer_.download(out, B_.advanced, V_ * sizeof(cplx), stream_);
 }
 
 void CartesianWorkspace::read_state(double* out) {
   if (!loaded_) throw Error(kState, "no state is loaded");
-  SP_HIP(hipStreamSynchronize(stream_));
-  SP_HIP(hipMemcpy(out, B_.y, V_ * sizeof(cplx), hipMemcpyDeviceToHost));
+  transfer_.download(out, B_.y, V_ * sizeof(cplx), stream_);
 }
 
 void CartesianWorkspace::export_state(const double* weight, bool optics, double* out) {

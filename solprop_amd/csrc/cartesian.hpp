@@ -25,6 +25,7 @@
 #include "field.hpp"
 #include "march.hpp"
 #include "propagator.hpp"
+#include "transfer.hpp"
 
 namespace sp {
 
@@ -82,6 +83,7 @@ class CartesianWorkspace final : public Propagator {
   std::vector<void*> allocations_;
   std::size_t device_bytes_ = 0;
   hipStream_t stream_ = nullptr;
+  Transfer transfer_;
   cplx *roots_t_ = nullptr, *roots_x_ = nullptr, *roots_y_ = nullptr;  // unit roots
   cplx* field_ = nullptr;  // the (y, x, t) samples the transforms and the response act on
   cplx *acc_ = nullptr, *prev_ = nullptr, *save_ = nullptr;

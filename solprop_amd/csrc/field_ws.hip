@@ -793,8 +793,7 @@ void FieldWorkspace::load(double z, const double* field) {
   const std::size_t CN = static_cast<std::size_t>(P_.C) * P_.N;
   pending_slot_ = -1;
   monitor_.reset(stream_);
-  SP_HIP(hipStreamSynchronize(stream_));
-  SP_HIP(hipMemcpy(B_.y, field, CN * sizeof(cplx), hipMemcpyHostToDevice));
+  transfer_.upload(B_.y, field, CN * sizeof(cplx), stream_);
   adams::Engine& engine = *this;
   march_ = std::make_unique<adams::March>(policy_, engine, host_, z, dz_init_);
   if (low_storage_) {
@@ -837,15 +836,13 @@ double FieldWorkspace::probe_trial(double z, double dz) {
 }
 
 void FieldWorkspace::read_trial(double* out) {
-  SP_HIP(hipStreamSynchronize(stream_));
-  SP_HIP(hipMemcpy(out, B_.advanced, sizeof(cplx) * P_.C * P_.N, hipMemcpyDeviceToHost));
+  transfer_.download(out, B_.advanced, sizeof(cplx) * P_.C * P_.N, stream_);
 }
 
 void FieldWorkspace::read_state(double* out) {
   if (!loaded_) throw Error(kState, "no state is loaded");
   flush();
-  SP_HIP(hipStreamSynchronize(stream_));
-  SP_HIP(hipMemcpy(out, B_.y, sizeof(cplx) * P_.C * P_.N, hipMemcpyDeviceToHost));
+  transfer_.download(out, B_.y, sizeof(cplx) * P_.C * P_.N, stream_);
 }
 
 void FieldWorkspace::export_state(const double* weight, bool optics, double* out) {

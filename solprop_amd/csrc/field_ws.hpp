@@ -16,6 +16,7 @@
 #include "propagator.hpp"
 #include "scalars.hpp"
 #include "stats.hpp"
+#include "transfer.hpp"
 
 namespace sp {
 
@@ -138,6 +139,7 @@ class FieldWorkspace final : public Propagator, private adams::Engine {
   std::vector<void*> allocations_;
   std::size_t device_bytes_ = 0;
   hipStream_t stream_ = nullptr;
+  Transfer transfer_;
   bool own_stream_ = true;
   FftPlan inv_plan_, fwd_plan_;
   cplx* scratch_ = nullptr;
