@@ -20,7 +20,7 @@ CSRC = HERE / "csrc"
 OUT = HERE / "libsolprop_mi355x.so"
 ARCH = "gfx950"
 
-HIP_SOURCES = ["fft.hip", "gemm.hip", "stage.hip", "field.hip", "workspace.hip", "field_ws.hip",
+HIP_SOURCES = ["fft.hip", "gemm.hip", "stage.hip", "env_stage.hip", "field.hip", "workspace.hip", "field_ws.hip",
                "stats.hip", "scan.hip", "fft_noalloc.hip",
                "fno.hip", "fno_tile.hip", "cartesian.hip"]
 HOST_SOURCES = ["capi.cpp", "session.cpp", "transfer.cpp"]

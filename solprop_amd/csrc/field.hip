@@ -2297,12 +2297,11 @@ void launch_quadrature_score(const cplx* fine, const cplx* coarse, long n, doubl
   check();
 }
 
-void launch_record_fetch(const AdamsRecord* host, AdamsRecord* device, int count,
-                         hipStream_t s) {
-  const int words = static_cast<int>(count * sizeof(AdamsRecord) / sizeof(unsigned long long));
+void launch_record_fetch(const void* host, void* device, std::size_t bytes, hipStream_t s) {
+  const int words = static_cast<int>(bytes / sizeof(unsigned long long));
   hipLaunchKernelGGL(record_fetch, dim3(1), dim3(kFetchThreads), 0, s,
-                     reinterpret_cast<const unsigned long long*>(host),
-                     reinterpret_cast<unsigned long long*>(device), words);
+                     static_cast<const unsigned long long*>(host),
+                     static_cast<unsigned long long*>(device), words);
   check();
 }
 

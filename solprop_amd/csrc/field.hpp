@@ -267,10 +267,6 @@ void launch_adams_commit(const DeviceProblem& P, const AdamsRecord* R, FieldBuff
 // one workgroup summing in a fixed order.
 void launch_quadrature_score(const cplx* fine, const cplx* coarse, long n, double* out,
                              hipStream_t s);
-// The upload of `count` records from pinned host memory (`host` as the device addresses
-// it) to `device`, as a kernel of one workgroup that reads them at system scope.
-void launch_record_fetch(const AdamsRecord* host, AdamsRecord* device, int count,
-                         hipStream_t s);
 void launch_adams_start(const DeviceProblem& P, const AdamsRecord* R, FieldBuffers B,
                         hipStream_t s);
 

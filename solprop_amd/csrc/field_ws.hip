@@ -444,7 +444,7 @@ void FieldWorkspace::enqueue_start() {
 void FieldWorkspace::enqueue(int key) {
   // The record's upload is the graph's first node: the host fills the pinned record,
   // then launches one graph.
-  launch_record_fetch(rec_host_dev_, rec_dev_, 1, stream_);
+  launch_record_fetch(rec_host_dev_, rec_dev_, sizeof(AdamsRecord), stream_);
   const int kind = key & 15;
   if (kind == kStart)
     enqueue_start();

@@ -35,6 +35,7 @@ Workspace::Workspace(const sp_problem_desc& d) {
   SP_CHECK(d.kind == 0, "the Runge-Kutta workspace runs the envelope route");
   SP_CHECK(d.method == 0, "the envelope route marches with the embedded Runge-Kutta pair");
   SP_CHECK(d.n_to >= 16 && (d.n_to & (d.n_to - 1)) == 0, "n_to must be a power of two >= 16");
+  SP_CHECK(d.n_to <= (1 << 24), "FFT length above 2^24 is not supported");
   SP_CHECK(d.n_t >= 4 && d.n_to % d.n_t == 0, "n_to must be a multiple of n_t");
   SP_CHECK(d.n_omega == d.n_t, "an envelope grid has n_omega = n_t bins");
   SP_CHECK(d.n_modes >= 1 && d.n_nodes == 1, "the envelope route runs one node");
@@ -78,7 +79,7 @@ Workspace::Workspace(const sp_problem_desc& d) {
   // The split collar changes the committed state after the trial: its last stage is no
   // longer the new state's first, and every stage is evaluated
   // (src/solprop/backends/numpy_ref/engines.py:99-178).
-  fsal_ = d.first_same_as_last != 0 && !split_;
+  fsal_ = d.first_same_as_last != 0 && !split_ && d.n_stages > 1;
 
   // Controller and landings (the run's policy, src/solprop/backends/records.py:227).
   auto& c = policy_.controller;
@@ -164,26 +165,56 @@ Workspace::Workspace(const sp_problem_desc& d) {
   recycled_ = device_alloc<cplx>(CN);
   einv_ = device_alloc<cplx>(CN);
   k_ = device_alloc<cplx>(CN * d.n_stages);
-  const std::size_t rows = in_stage_ ? 2 * C : C;
-  fine_ = device_alloc<cplx>(rows * T);
-  scratch_ = device_alloc<cplx>(rows * T);
-  fine_plan_.init(T, C);
-  if (in_stage_) forward_plan_.init(T, rows);
+  fine_ = device_alloc<cplx>((in_stage_ ? 2 : 1) * static_cast<std::size_t>(T));
+  scratch_ = device_alloc<cplx>(T);
   if (split_) coarse_plan_.init(N, C);
   if (d.n_raman) {
-    drive_ = device_alloc<cplx>(T);
-    H_ = device_alloc<cplx>(T + 1);
-    const auto roots = unit_roots(2 * static_cast<std::size_t>(T));
-    roots2T_ = device_copy(roots.data(), roots.size());
+    H_ = device_alloc<cplx>(T);
     raman_plan_.init(T, 1);
   }
-  n_partial_blocks_ = static_cast<int>(accept_blocks(P_));
-  partials_ = device_alloc<double>(3 * static_cast<std::size_t>(n_partial_blocks_));
+  int m = 0;
+  while ((1 << m) < T) ++m;
+  env_.log2n1 = m / 2;
+  env_.log2n2 = m - m / 2;
+  auto roots = [&](int log2n) {
+    const auto w = unit_roots(std::size_t{1} << log2n);
+    return device_copy(w.data(), w.size());
+  };
+  env_.roots_l[0] = roots(env_.log2n1);
+  env_.roots_l[1] = env_.log2n2 == env_.log2n1 ? env_.roots_l[0] : roots(env_.log2n2);
+  if (d.n_raman) {
+    env_.roots = raman_plan_.roots();
+    // W_4T^t over its quadrant, t < T.
+    std::vector<cplx> twist(T);
+    const long double turn = 6.283185307179586476925286766559005768L / (4.0L * T);
+    for (int t = 0; t < T; ++t) {
+      const bool low = 2 * t <= T;
+      const long double angle = turn * (low ? t : T - t);
+      const long double c = std::cos(angle), s = std::sin(angle);
+      twist[t] = make(static_cast<double>(low ? c : s), -static_cast<double>(low ? s : c));
+    }
+    env_.twist = device_copy(twist.data(), twist.size());
+    env_.field = device_alloc<cplx>(T);
+    env_.kernel = H_;
+  } else {
+    env_.roots = roots(m);
+  }
+  env_.y = y_;
+  env_.k = k_;
+  env_.einv = einv_;
+  env_.adv = adv_;
+  env_.recycled = recycled_;
+  env_.P = P_;
+  n_partial_blocks_ = static_cast<int>(env_accept_blocks(env_));
   rec_dev_ = device_alloc<TrialRecord>(1);
+  env_.R = rec_dev_;
   SP_HIP(hipHostMalloc(reinterpret_cast<void**>(&rec_host_), sizeof(TrialRecord)));
   std::memset(rec_host_, 0, sizeof(TrialRecord));
+  SP_HIP(hipHostGetDevicePointer(const_cast<void**>(&rec_host_dev_), rec_host_, 0));
   SP_HIP(hipHostMalloc(reinterpret_cast<void**>(&partials_host_),
-                       3 * sizeof(double) * n_partial_blocks_));
+                       3 * sizeof(double) * n_partial_blocks_, hipHostMallocMapped));
+  SP_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&env_.partials), partials_host_, 0));
+  SP_HIP(hipEventCreateWithFlags(&done_, hipEventDisableTiming));
   SP_HIP(hipEventCreate(&ev0_));
   SP_HIP(hipEventCreate(&ev1_));
 }
@@ -194,6 +225,7 @@ Workspace::~Workspace() {
   for (void* p : allocations_) (void)hipFree(p);
   if (rec_host_) (void)hipHostFree(rec_host_);
   if (partials_host_) (void)hipHostFree(partials_host_);
+  if (done_) (void)hipEventDestroy(done_);
   if (ev0_) (void)hipEventDestroy(ev0_);
   if (ev1_) (void)hipEventDestroy(ev1_);
   if (stream_) (void)hipStreamDestroy(stream_);
@@ -220,28 +252,35 @@ void Workspace::fill_record(double z, double dz) {
 }
 
 void Workspace::enqueue_raman_kernel(int stage) {
-  launch_raman_kernel_fill(P_, rec_dev_, stage, drive_, stream_);
-  raman_plan_.exec(drive_, scratch_, -1, stream_);
-  launch_raman_kernel_post(drive_, H_, roots2T_, P_.T, P_.dt_fine, stream_);
+  launch_env_raman_kernel(env_, stage, H_, stream_);
+  raman_plan_.exec(H_, scratch_, -1, stream_);
 }
 
-void Workspace::enqueue_stage(int stage, bool finish_previous) {
-  // The previous stage's finish rides in this stage's entry, and the last stage's in the
-  // step's acceptance.
-  if (finish_previous)
-    launch_rk_finish_entry(P_, rec_dev_, y_, k_, fine_, einv_, stage, stream_);
-  else
-    launch_rk_entry_envelope(P_, rec_dev_, y_, k_, fine_, einv_, stage, stream_);
-  fine_plan_.exec(fine_, scratch_, +1, stream_);
-  if (P_.n_raman) {
-    if (raman_dynamic_) enqueue_raman_kernel(stage);
-    launch_env_raman_drive(P_, rec_dev_, fine_, drive_, stage, stream_);
-    raman_plan_.exec(drive_, scratch_, -1, stream_);
-    launch_raman_product(drive_, H_, roots2T_, P_.T, 1, stream_);
-    raman_plan_.exec(drive_, scratch_, +1, stream_);
+void Workspace::enqueue_stage(int stage, bool finish_previous, bool commit, bool recycle) {
+  // The Raman kernel's transform uses `scratch_`, which is free between a response and the
+  // finish or entry after it.
+  if (P_.n_raman && raman_dynamic_) enqueue_raman_kernel(stage);
+  EnvStage a = env_;
+  a.in = fine_;
+  a.out = scratch_;
+  if (finish_previous) {
+    launch_env_finish(a, stage, stream_);
+  } else {
+    a.commit = commit ? 1 : 0;
+    a.recycle = recycle ? 1 : 0;
+    launch_env_entry(a, stage, stream_);
   }
-  launch_env_response(P_, rec_dev_, fine_, drive_, stage, stream_);
-  (in_stage_ ? forward_plan_ : fine_plan_).exec(fine_, scratch_, -1, stream_);
+  if (P_.n_raman) {
+    a.in = scratch_;
+    a.out = fine_;
+    launch_env_drive(a, stage, stream_);
+    a.in = fine_;
+    a.out = scratch_;
+    launch_env_product(a, stage, stream_);
+  }
+  a.in = scratch_;
+  a.out = fine_;
+  launch_env_response(a, stage, stream_);
 }
 
 void Workspace::enqueue_commit(const TrialRecord* R, double dz) {
@@ -262,19 +301,22 @@ void Workspace::enqueue_commit(const TrialRecord* R, double dz) {
 }
 
 void Workspace::enqueue_trial(bool commit, Stage0 mode) {
-  const long CN = static_cast<long>(P_.C) * P_.N;
-  if (commit) enqueue_commit(rec_dev_, 0.0);
-  if (mode == kCopyRecycled) launch_copy_points(recycled_, k_, CN, stream_);
+  launch_record_fetch(rec_host_dev_, rec_dev_, sizeof(TrialRecord), stream_);
+  // Under the split-step absorber the commit is launches of its own (the collar acts on
+  // the committed field), else the first entry commits bin by bin.
+  if (commit && split_) enqueue_commit(rec_dev_, 0.0);
   const int first = mode == kEvaluate ? 0 : 1;
-  for (int i = first; i < P_.n_stages; ++i) enqueue_stage(i, i > first);
-  launch_rk_accept(P_, rec_dev_, y_, k_, adv_, recycled_, partials_, fine_, einv_, stream_);
+  for (int i = first; i < P_.n_stages; ++i)
+    enqueue_stage(i, i > first, commit && !split_, mode == kCopyRecycled);
+  EnvStage a = env_;
+  a.in = fine_;
+  launch_env_accept(a, stream_);
 }
 
 double Workspace::finish_trial() {
-  SP_HIP(hipMemcpyAsync(partials_host_, partials_, 3 * sizeof(double) * n_partial_blocks_,
-                        hipMemcpyDeviceToHost, stream_));
   if (profile_) SP_HIP(hipEventRecord(ev1_, stream_));
-  SP_HIP(hipStreamSynchronize(stream_));
+  SP_HIP(hipEventRecord(done_, stream_));
+  wait_event(done_);
   if (profile_) {
     float ms = 0.0f;
     SP_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
@@ -305,8 +347,6 @@ double Workspace::trial(double z, double dz, bool full) {
     else if (!commit && k0_valid_ && k0_z_ == z)
       mode = kKeep;
   }
-  SP_HIP(hipMemcpyAsync(rec_dev_, rec_host_, sizeof(TrialRecord), hipMemcpyHostToDevice,
-                        stream_));
   if (profile_) SP_HIP(hipEventRecord(ev0_, stream_));
   const int key = (commit ? 4 : 0) + static_cast<int>(mode);
   if (use_graphs_) {
@@ -510,8 +550,7 @@ sp_counters Workspace::counters() const {
   c.evaluations = evaluations_;
   c.accepted = accepted_;
   c.graph_launches = graph_launches_;
-  c.device_bytes = static_cast<long>(device_bytes_ + fine_plan_.bytes() + raman_plan_.bytes() +
-                                     forward_plan_.bytes() + coarse_plan_.bytes() +
+  c.device_bytes = static_cast<long>(device_bytes_ + raman_plan_.bytes() + coarse_plan_.bytes() +
                                      (stats_ ? stats_->bytes() : 0));
   return c;
 }

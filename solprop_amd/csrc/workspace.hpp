@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "device.hpp"
+#include "kernels.hpp"
 #include "fft.hpp"
 #include "march.hpp"
 #include "propagator.hpp"
@@ -52,8 +53,9 @@ class Workspace final : public Propagator {
   T* device_alloc(std::size_t n);
   void fill_record(double z, double dz);
   void enqueue_trial(bool commit, Stage0 mode);
-  // One stage; with `finish_previous` its entry also finishes the stage before it.
-  void enqueue_stage(int stage, bool finish_previous);
+  // One stage; `finish_previous`: its entry also finishes the stage before it, else it may
+  // first commit the held trial (`commit`) and take its last stage as k[0] (`recycle`).
+  void enqueue_stage(int stage, bool finish_previous, bool commit, bool recycle);
   void enqueue_raman_kernel(int stage);
   void ensure_committed();
   // The commit of the held trial: the band mask and, under the split-step absorber, the
@@ -65,10 +67,9 @@ class Workspace final : public Propagator {
   std::vector<void*> allocations_;
   std::size_t device_bytes_ = 0;
   hipStream_t stream_ = nullptr;
-  FftPlan fine_plan_, raman_plan_;
-  // The forward transform over the polarisation's rows and the in-stage absorber's, and
-  // the coarse grid's transform for the split-step absorber.
-  FftPlan forward_plan_, coarse_plan_;
+  FftPlan raman_plan_;
+  EnvStage env_{};
+  FftPlan coarse_plan_;  // for the split-step absorber
   bool in_stage_ = false, split_ = false;
   std::unique_ptr<PlaneStatistics> stats_;  // built at the first statistics call
   MonitorBuffers monitor_;
@@ -80,12 +81,13 @@ class Workspace final : public Propagator {
   bool fsal_ = false, raman_dynamic_ = false;
   // Device buffers.
   cplx *y_ = nullptr, *adv_ = nullptr, *recycled_ = nullptr, *einv_ = nullptr, *k_ = nullptr;
-  cplx *fine_ = nullptr, *scratch_ = nullptr, *drive_ = nullptr, *H_ = nullptr;
-  cplx* roots2T_ = nullptr;
-  double* partials_ = nullptr;
+  // The stage kernels' two buffers (what a response leaves, with the absorber's row, and
+  // what the others do), and the Raman kernel's transform.
+  cplx *fine_ = nullptr, *scratch_ = nullptr, *H_ = nullptr;
   TrialRecord* rec_dev_ = nullptr;
-  TrialRecord* rec_host_ = nullptr;
-  double* partials_host_ = nullptr;
+  TrialRecord* rec_host_ = nullptr;       // pinned
+  const void* rec_host_dev_ = nullptr;    // as the device addresses it
+  double* partials_host_ = nullptr;       // mapped: the acceptance's sums as they are stored
   int n_partial_blocks_ = 0;
   // Graphs keyed by (commit, stage-0 mode).
   std::map<int, hipGraphExec_t> graphs_;
@@ -99,7 +101,7 @@ class Workspace final : public Propagator {
   // Counters and timing.
   long trials_ = 0, evaluations_ = 0, accepted_ = 0, graph_launches_ = 0;
   bool profile_ = false;
-  hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
+  hipEvent_t ev0_ = nullptr, ev1_ = nullptr, done_ = nullptr;
   double time_total_ms_ = 0.0;
   long timed_ = 0;
 };
