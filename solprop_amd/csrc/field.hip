@@ -430,6 +430,43 @@ __device__ inline double band_filter(const PlasmaTable& pt, const double* window
   return f;
 }
 
+// A node's window where a wave holds one for each of its nodes: kBandSpan samples and the
+// K reflections past the grid's end that the last tile's lanes hold.
+constexpr int kWindowRow = kBandSpan + kMaxBandHalf;
+
+// The filter and the inclusive scan of N nodes side by side, so that one's LDS reads and
+// cross-lane moves hide the others' latency; each node's sums are those of band_filter
+// and wave_scan.
+template <int N>
+__device__ inline void band_filter_nodes(const PlasmaTable& pt, const double* windows, int lane,
+                                         double (&f)[N]) {
+  const int K = pt.n_taps - 1;
+  const double* y = windows + K + lane;
+#pragma unroll
+  for (int i = 0; i < N; ++i) f[i] = pt.taps[0] * y[i * kWindowRow];
+#pragma unroll 1
+  for (int k = 1; k <= K; ++k)
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      f[i] = f[i] + pt.taps[k] * (y[i * kWindowRow - k] + y[i * kWindowRow + k]);
+}
+
+template <int Ctrl, int RowMask, bool Bound, int N>
+__device__ inline void scan_step(double (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = v[i] + dpp_move<Ctrl, RowMask, Bound>(v[i]);
+}
+
+template <int N>
+__device__ inline void wave_scan_nodes(double (&v)[N]) {
+  scan_step<0x111, 0xf, true>(v);
+  scan_step<0x112, 0xf, true>(v);
+  scan_step<0x114, 0xf, true>(v);
+  scan_step<0x118, 0xf, true>(v);
+  scan_step<0x142, 0xa, false>(v);
+  scan_step<0x143, 0xc, false>(v);
+}
+
 // The rate at node q and sample t of the grid.
 template <int C>
 __device__ inline double rate_sample(const DeviceProblem& P, const PlasmaTable& pt,
@@ -499,17 +536,6 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Whether a node's whole filter window is zero: every lane's own value and the node's 2K
-// halo values (wave-uniform). With a positive centre tap the filter of such a window is
-// +0.0 at every lane, and so are the trapezoid increments and their scans, so a pass
-// may store those zeros without forming them (the same bits): away from the pulse the
-// rate vanishes, and before it the free-current integrand.
-__device__ inline bool window_is_zero(const PlasmaTable& pt, double own,
-                                      const double* halo_row, int lane) {
-  const double h = lane < 2 * (pt.n_taps - 1) ? halo_row[lane] : 0.0;
-  return pt.taps[0] > 0.0 && __ballot(own != 0.0 || h != 0.0) == 0;
-}
-
 // The band passes run each wave's nodes as the trapezoid passes do (modal fields of the
 // lane's sample held in registers across them), with the samples a node needs beyond
 // its own lanes evaluated first for every node of the wave: the filter's halo of 2K
@@ -523,24 +549,24 @@ __device__ inline int extra_sample(int tile, int K, int T, int h) {
   return h < 2 * K ? halo_sample(tile, K, h) : T + (h - 2 * K);
 }
 
-// Up to four modes the band passes ask for six (rate) and eight (current) waves a SIMD:
-// at most 80 and 64 VGPRs, with no scratch; more modes hold more registers and ask for
-// fewer waves, again with no scratch.
+// Up to four modes the band passes ask for six (rate) and eight (unfused current) waves a
+// SIMD, at most 80 and 64 VGPRs, with no scratch; more modes hold more registers and ask
+// for fewer waves, again with no scratch. The fused current pass asks for five (96 VGPRs;
+// at six it spills from four modes on, and gains nothing below).
 
 // Pass A under the band rule: the raw rate stored for the owned samples, the filtered
 // rate's trapezoid increments scanned, the within-tile exposure stored and the tile's
 // sum.
-// LDS a band pass's workgroup holds: each wave's window and its nodes' extra samples.
-template <int NPW>
-struct BandLdsN {
+// LDS the unfused current pass's workgroup holds: each wave's window and its nodes' extra
+// samples.
+struct BandLds {
   double windows[kNodeWaves][kBandSpan];
-  double halos[kNodeWaves][NPW * kBandSlots];
+  double halos[kNodeWaves][kNodesPerWave * kBandSlots];
 };
-using BandLds = BandLdsN<kNodesPerWave>;
 
 // The nodes a wave of the rate pass runs: on the modal route half as many as the other
 // band passes, for more waves to hide the loads' latency (at 2^14 samples and 128 nodes
-// 15.7 us against 17.5 with four and 19.3 with one); on the dense route (C = 0) as many
+// 13.4 us, 15.6 with its nodes one after another); on the dense route (C = 0) as many
 // (26.8 us against 24.5 with two at the radial grid).
 template <int C>
 constexpr int rate_nodes_per_wave() {
@@ -554,69 +580,86 @@ inline int rate_groups(int Q) {
 
 template <int C, int NPW = kNodesPerWave>
 __device__ __forceinline__ void rate_band_body(const DeviceProblem& P, const PlasmaTable& pt,
-                                      const FieldBuffers& B, int tile, int group, double* table,
-                                      BandLdsN<NPW>& lds, bool sparse) {
-  auto& windows = lds.windows;
-  auto& halos = lds.halos;
-  (void)table;
+                                      const FieldBuffers& B, int tile, int group,
+                                      double* lds, bool sparse) {
   // The rate table is read through the vector caches: most workgroups lie where the field
   // is below the table's threshold and never read it, so no workgroup waits to stage it.
   const double* coefficients = B.rate_c;
   const int T = P.T, tiles = scan_tiles(T), K = pt.n_taps - 1, H = 2 * K;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int t = tile * kTileSpan + lane;
   const bool stores = t < T && (lane < kTileSpan || t == T - 1);
   const bool step = lane < kTileSpan && t + 1 < T;
-  double* window = windows[wave];
-  double* halo = halos[wave];
+  double* own = lds + wave * (NPW * kWindowRow);  // a window a node
   const int q0 = group * kNodeWaves * NPW + wave;
-  const int S = H + (tile == tiles - 1 ? K : 0);  // extra samples a node needs
-  // The lane's own modal fields first, so that their loads overlap the halo's (up to four
-  // modes: more held across the halo would spill).
+  const bool last = tile == tiles - 1;
+  const int S = H + (last ? K : 0);  // extra samples a node needs
+  const int tc = min(t, T - 1);
   double am[held(C)];
-  if constexpr (C <= 4) load_modal<C>(B, T, t, am);
+  load_modal<C>(B, T, tc, am);
+  const bool inner = tile * kTileSpan >= K && tile * kTileSpan + kWave - 1 + K <= T - 1;
   for (int idx = lane; idx < NPW * S; idx += kWave) {
     const int i = idx / S, h = idx - i * S;
-    const int q = q0 + i * kNodeWaves;
-    double v = 0.0;
-    if (q < P.Q) {
-      auto sample = [&](int u) { return rate_sample<C>(P, pt, coefficients, B, q, u); };
-      v = reflected(T, K, extra_sample(tile, K, T, h), sample);
-    }
-    halo[i * kBandSlots + h] = v;
+    const int q = min(q0 + i * kNodeWaves, P.Q - 1);
+    auto sample = [&](int u) { return rate_sample<C>(P, pt, coefficients, B, q, u); };
+    const int u = extra_sample(tile, K, T, h);
+    own[i * kWindowRow + (h < H ? halo_slot(K, h) : kBandSpan + h - H)] =
+        inner ? sample(u) : reflected(T, K, u, sample);
   }
+  double e[NPW], w[NPW];
+#pragma unroll
+  for (int i = 0; i < NPW; ++i) e[i] = field_at<C>(P, B, am, min(q0 + i * kNodeWaves, P.Q - 1), tc);
+#pragma unroll
+  for (int i = 0; i < NPW; ++i) w[i] = rate_of(fabs(e[i]), pt, coefficients);
   wave_sync();
-  if constexpr (C > 4) load_modal<C>(B, T, t, am);
+  if (last) {  // the last tile's lanes past the end: their reflections
+#pragma unroll
+    for (int i = 0; i < NPW; ++i)
+      if (t >= T) w[i] = t - T < K ? own[i * kWindowRow + kBandSpan + (t - T)] : 0.0;
+  }
+  // Which nodes' whole filter windows are zero: every lane's own value and the 2K halo
+  // values. With a positive centre tap the filter of such a window is +0.0 at every lane,
+  // and so are the trapezoid increments and their scans, so the pass may store those zeros
+  // without forming them: away from the pulse the rate vanishes.
+  unsigned busy = 0;
+#pragma unroll
   for (int i = 0; i < NPW; ++i) {
-    const int q = q0 + i * kNodeWaves;
-    if (q >= P.Q) break;  // uniform across the wave, and so for every later node
-    double w = 0.0;
-    if (t < T)
-      w = rate_of(fabs(field_at<C>(P, B, am, q, t)), pt, coefficients);
-    else if (t - T < K)  // the last tile's lanes past the end: their reflections
-      w = halo[i * kBandSlots + H + (t - T)];
-    const long row = static_cast<long>(q) * T;
-    const bool zero = window_is_zero(pt, w, halo + i * kBandSlots, lane);
-    if (B.zero_tiles && lane == 0) B.zero_tiles[static_cast<long>(q) * tiles + tile] = zero;
-    if (stores && !(zero && sparse)) B.rate[row + t] = w;
-    if (zero) {
-      if (lane == kTileSpan - 1) B.tile_x[static_cast<long>(q) * tiles + tile] = 0.0;
-      if (stores && !sparse) B.x_local[row + t] = 0.0;
-      continue;
-    }
-    wave_sync();  // the previous node's window has been read
-    window[K + lane] = w;
-    if (lane < H) window[halo_slot(K, lane)] = halo[i * kBandSlots + lane];
+    const double h = lane < H ? own[i * kWindowRow + halo_slot(K, lane)] : 0.0;
+    if (!(pt.taps[0] > 0.0) || __ballot(w[i] != 0.0 || h != 0.0) != 0) busy |= 1u << i;
+  }
+  double excl[NPW], incl[NPW];
+#pragma unroll
+  for (int i = 0; i < NPW; ++i) excl[i] = incl[i] = 0.0;
+  if (busy != 0) {
+#pragma unroll
+    for (int i = 0; i < NPW; ++i) own[i * kWindowRow + K + lane] = w[i];
     wave_sync();
     // Cross-lane moves with every lane of the wave active: a lane masked off reads as
     // zero to its neighbours.
-    const double y = band_filter(pt, window, lane);
-    const double y_next = from_next_lane(y);
-    const double inc = step ? (P.dt_fine * (y_next + y)) / 2.0 : 0.0;
-    const double incl = wave_scan(inc);
-    const double excl = from_previous_lane(incl);
-    if (lane == kTileSpan - 1) B.tile_x[static_cast<long>(q) * tiles + tile] = incl;
-    if (stores) B.x_local[row + t] = excl;
+    double y[NPW];
+    band_filter_nodes<NPW>(pt, own, lane, y);
+#pragma unroll
+    for (int i = 0; i < NPW; ++i) {
+      const double y_next = from_next_lane(y[i]);
+      incl[i] = step ? (P.dt_fine * (y_next + y[i])) / 2.0 : 0.0;
+    }
+    wave_scan_nodes<NPW>(incl);
+#pragma unroll
+    for (int i = 0; i < NPW; ++i) excl[i] = from_previous_lane(incl[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < NPW; ++i) {
+    const int q = q0 + i * kNodeWaves;
+    if (q >= P.Q) break;  // uniform across the wave, and so for every later node
+    const bool zero = !(busy & (1u << i));
+    const long row = static_cast<long>(q) * T, at = static_cast<long>(q) * tiles + tile;
+    if (B.zero_tiles && lane == 0) B.zero_tiles[at] = zero;
+    if (lane == kTileSpan - 1) B.tile_x[at] = zero ? 0.0 : incl[i];
+    if (stores && !(zero && sparse)) {
+      B.rate[row + t] = w[i];
+      B.x_local[row + t] = zero ? 0.0 : excl[i];
+    }
   }
 }
 
@@ -624,9 +667,8 @@ template <int C>
 __global__ void __launch_bounds__(kWave * kNodeWaves)
     __attribute__((amdgpu_waves_per_eu(C <= 4 ? 6 : 4)))
     plasma_rate_band(DeviceProblem P, PlasmaTable pt, FieldBuffers B, int sparse) {
-  __shared__ BandLdsN<rate_nodes_per_wave<C>()> lds;
-  rate_band_body<C, rate_nodes_per_wave<C>()>(P, pt, B, blockIdx.x, blockIdx.y, nullptr, lds,
-                                              sparse != 0);
+  __shared__ double lds[kNodeWaves * rate_nodes_per_wave<C>() * kWindowRow];
+  rate_band_body<C, rate_nodes_per_wave<C>()>(P, pt, B, blockIdx.x, blockIdx.y, lds, sparse != 0);
 }
 
 // Pass C under the band rule: the free-current integrand (the fraction from the stored
@@ -715,20 +757,32 @@ __global__ void __launch_bounds__(kWave * kNodeWaves)
 // band pass (either rule: the trapezoid is one tap), then at the lane's sample the
 // polarisation (Kerr and Raman) and the current F_local + I_p W (1 - f) E / |E|², each
 // projected onto the modes and summed over the wave's nodes in order, then over the
-// waves in order (`red`, 2C rows of kWave for each wave). The group's rows of B.group_streams receive
+// waves in order. The group's rows of B.group_streams receive
 // the sums at the tile's owned samples, and B.tile_p its nodes' free-current tile
 // totals projected onto the modes (nodes in order; `totals` holds kNodesPerGroup).
+// What bounds the pass is latency: a wave's chain of loads, exponentials, LDS fences and
+// scans. Every load is therefore issued before the first fence (node indices are made
+// wave-uniform, so that the synthesis and projection rows are scalar loads), and the
+// wave's four nodes go through the filter and the scans side by side behind one fence,
+// each node with a window of its own. At 2^14 samples, four modes and 128 nodes 26.4 us (27.8
+// with the nodes one after another); over a scan's 48 uneven instances 588 us (636), the rate
+// pass done the same way 308 us (357).
 template <int C>
+__host__ __device__ constexpr int current_lds_row() {  // doubles of LDS a wave holds
+  constexpr int windows = kNodesPerWave * kWindowRow;
+  return windows > C * kWave ? windows : C * kWave;
+}
+
+template <int C, int ROW>
 __device__ __forceinline__ void current_response_body(const DeviceProblem& P,
                                                       const PlasmaTable& pt,
                                                       const AdamsRecord* __restrict__ R,
                                                       const FieldBuffers& B, int tile,
-                                                      int group, BandLds& lds, double* red,
-                                                      double* totals) {
-  auto& windows = lds.windows;
-  auto& halos = lds.halos;
+                                                      int group, double* lds, double* totals) {
+  constexpr int NPW = kNodesPerWave;
   const int T = P.T, tiles = scan_tiles(T), K = pt.n_taps - 1, H = 2 * K;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int t = tile * kTileSpan + lane;
   const int owner = min(t / kTileSpan, tiles - 1);
   const bool stores = t < T && (lane < kTileSpan || t == T - 1);
@@ -736,117 +790,132 @@ __device__ __forceinline__ void current_response_body(const DeviceProblem& P,
   const double f0 = R->preionisation;
   const double density = R->density;
   const double kerr = P.has_kerr ? P.kerr_coefficient * density : 0.0;
-  double* window = windows[wave];
-  double* halo = halos[wave];
+  double* own = lds + wave * ROW;  // the wave's windows, then its rows of the projections
   const int base = group * kNodesPerGroup;
   const int q0 = base + wave;
-  const int S = H + (tile == tiles - 1 ? K : 0);  // extra samples a node needs
-  // Every node's exposure and rate at the lane's sample are loaded before the halo is
-  // evaluated, so that their latency overlaps it (the node loop's LDS fences would
-  // otherwise hold each node's loads until the previous node is done).
+  const bool last = tile == tiles - 1;
+  const int S = H + (last ? K : 0);  // extra samples a node needs
   // A tile the rate pass flagged holds no stores: its rate and within-tile exposure are
   // zero, and the exposure there is the tile's offset (x + 0.0 is x).
   // No load sits under a branch (a branch would make each wait for the one before): the
   // flags and offsets are loaded from clamped addresses, all together; then the stored
   // tiles' entries, where a flagged tile reads a constant zero instead.
   const int tc = min(t, T - 1);
-  unsigned char zero[kNodesPerWave];
-  double xs[kNodesPerWave], ws[kNodesPerWave];
+  int node[NPW];
+  unsigned char zero[NPW];
+  double xs[NPW], ws[NPW];
 #pragma unroll
-  for (int i = 0; i < kNodesPerWave; ++i) {
-    const long tq = static_cast<long>(min(q0 + i * kNodeWaves, P.Q - 1)) * tiles + owner;
+  for (int i = 0; i < NPW; ++i) {
+    node[i] = min(q0 + i * kNodeWaves, P.Q - 1);
+    const long tq = static_cast<long>(node[i]) * tiles + owner;
     zero[i] = B.zero_tiles[tq];
     xs[i] = B.tile_x[tq];
   }
+  double am[C];
+  load_modal<C>(B, T, tc, am);
 #pragma unroll
-  for (int i = 0; i < kNodesPerWave; ++i) {
-    const int q = q0 + i * kNodeWaves;
-    const bool here = q < P.Q && t < T;
-    const long at = static_cast<long>(min(q, P.Q - 1)) * T + tc;
+  for (int i = 0; i < NPW; ++i) {
+    const long at = static_cast<long>(node[i]) * T + tc;
     const double* x_at = zero[i] ? &kZeroSample : B.x_local + at;
     const double* w_at = zero[i] ? &kZeroSample : B.rate + at;
     const double local = *x_at, w = *w_at;
-    xs[i] = here ? xs[i] + local : 0.0;  // a flagged tile's offset plus 0.0
-    ws[i] = here ? w : 0.0;
+    xs[i] = t < T ? xs[i] + local : 0.0;  // a flagged tile's offset plus 0.0
+    ws[i] = t < T ? w : 0.0;
   }
-  for (int idx = lane; idx < kNodesPerWave * S; idx += kWave) {
+  // The extra samples, straight into the nodes' windows (the reflections past the grid's
+  // end after them). Only the tiles at the grid's ends reflect.
+  bool busy = false;
+  const bool inner = tile * kTileSpan >= K && tile * kTileSpan + kWave - 1 + K <= T - 1;
+  for (int idx = lane; idx < NPW * S; idx += kWave) {
     const int i = idx / S, h = idx - i * S;
-    const int q = q0 + i * kNodeWaves;
-    double v = 0.0;
-    if (q < P.Q) {
-      auto sample = [&](int u) { return current_sample_sparse<C>(P, B, q, u, f0, tiles); };
-      v = reflected(T, K, extra_sample(tile, K, T, h), sample);
-    }
-    halo[i * kBandSlots + h] = v;
+    const int q = min(q0 + i * kNodeWaves, P.Q - 1);
+    auto sample = [&](int u) { return current_sample_sparse<C>(P, B, q, u, f0, tiles); };
+    const int u = extra_sample(tile, K, T, h);
+    const double v = inner ? sample(u) : reflected(T, K, u, sample);
+    busy = busy || v != 0.0;
+    own[i * kWindowRow + (h < H ? halo_slot(K, h) : kBandSpan + h - H)] = v;
   }
-  wave_sync();
-  double am[held(C)];
-  load_modal<C>(B, T, t, am);
+  double f[NPW], e[NPW], y[NPW];
+#pragma unroll
+  for (int i = 0; i < NPW; ++i) {
+    f[i] = fraction_of(f0, xs[i] > 0.0 ? xs[i] : 0.0);
+    e[i] = synthesise_at<C>(P.synthesis + static_cast<long>(node[i]) * C, am);
+    y[i] = (f[i] * P.plasma_cmr) * e[i];
+  }
+  if (last) {  // the last tile's lanes past the end: nothing, then their reflections
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < NPW; ++i)
+      if (t >= T) {
+        f[i] = e[i] = 0.0;
+        y[i] = t - T < K ? own[i * kWindowRow + kBandSpan + (t - T)] : 0.0;
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < NPW; ++i) busy = busy || y[i] != 0.0;
+  // Before the pulse the integrand vanishes: the scan is zero, and a zero of either sign
+  // leaves the projections as they are.
+  double local[NPW], incl[NPW];
+#pragma unroll
+  for (int i = 0; i < NPW; ++i) local[i] = incl[i] = 0.0;
+  if (!(pt.taps[0] > 0.0) || __ballot(busy) != 0) {
+#pragma unroll
+    for (int i = 0; i < NPW; ++i) own[i * kWindowRow + K + lane] = y[i];
+    wave_sync();
+    // Cross-lane moves with every lane of the wave active (see the rate pass).
+    double yf[NPW];
+    band_filter_nodes<NPW>(pt, own, lane, yf);
+#pragma unroll
+    for (int i = 0; i < NPW; ++i) {
+      const double y_next = from_next_lane(yf[i]);
+      incl[i] = step ? (P.dt_fine * (y_next + yf[i])) / 2.0 : 0.0;
+    }
+    wave_scan_nodes<NPW>(incl);
+#pragma unroll
+    for (int i = 0; i < NPW; ++i) local[i] = from_previous_lane(incl[i]);
+  }
   double acc_p[C], acc_c[C];
 #pragma unroll
   for (int m = 0; m < C; ++m) acc_p[m] = acc_c[m] = 0.0;
 #pragma unroll
-  for (int i = 0; i < kNodesPerWave; ++i) {
-    const int q = q0 + i * kNodeWaves;
-    if (q >= P.Q) break;  // uniform across the wave, and so for every later node
-    double f = 0.0, e = 0.0, y = 0.0;
-    if (t < T) {
-      const double x = xs[i];
-      f = fraction_of(f0, x > 0.0 ? x : 0.0);
-      e = field_at<C>(P, B, am, q, t);
-      y = (f * P.plasma_cmr) * e;
-    } else if (t - T < K) {  // the last tile's lanes past the end: their reflections
-      y = halo[i * kBandSlots + H + (t - T)];
+  for (int i = 0; i < NPW; ++i) {
+    if (q0 + i * kNodeWaves >= P.Q) break;  // uniform, and so for every later node
+    if (lane == kTileSpan - 1) totals[i * kNodeWaves + wave] = incl[i];
+    const double w = ws[i];
+    const double squared = fabs(e[i]) * fabs(e[i]);
+    double loss = 0.0;
+    if (w > 0.0 && squared > 0.0) loss = (P.plasma_ip * w * (1.0 - f[i])) / squared;
+    const double current = local[i] + loss * e[i];
+    double pol = (kerr * (e[i] * e[i])) * e[i];
+    if (P.n_raman > 0) {
+      const double* conv = reinterpret_cast<const double*>(B.raman_drive);
+      pol = pol + ((P.raman_epsilon0 * density) * e[i]) * (conv[2L * node[i] * T + tc] * P.inv_2T);
     }
-    // Before the pulse the integrand vanishes: the scan is zero, and a zero of either sign
-    // leaves the projections as they are.
-    double local = 0.0, incl = 0.0;
-    if (!window_is_zero(pt, y, halo + i * kBandSlots, lane)) {
-      wave_sync();  // the previous node's window has been read
-      window[K + lane] = y;
-      if (lane < H) window[halo_slot(K, lane)] = halo[i * kBandSlots + lane];
-      wave_sync();
-      // Cross-lane moves with every lane of the wave active (see the rate pass).
-      const double yf = band_filter(pt, window, lane);
-      const double y_next = from_next_lane(yf);
-      const double inc = step ? (P.dt_fine * (y_next + yf)) / 2.0 : 0.0;
-      incl = wave_scan(inc);
-      local = from_previous_lane(incl);
-    }
-    if (lane == kTileSpan - 1) totals[i * kNodeWaves + wave] = incl;
-    if (t < T) {
-      const double w = ws[i];
-      const double squared = fabs(e) * fabs(e);
-      double loss = 0.0;
-      if (w > 0.0 && squared > 0.0) loss = (P.plasma_ip * w * (1.0 - f)) / squared;
-      const double current = local + loss * e;
-      double pol = (kerr * (e * e)) * e;
-      if (P.n_raman > 0) {
-        const double* conv = reinterpret_cast<const double*>(B.raman_drive);
-        pol = pol + ((P.raman_epsilon0 * density) * e) * (conv[2L * q * T + t] * P.inv_2T);
-      }
 #pragma unroll
-      for (int m = 0; m < C; ++m) {
-        const double wmq = P.projection[static_cast<long>(m) * P.Q + q];
-        acc_p[m] = acc_p[m] + wmq * pol;
-        acc_c[m] = acc_c[m] + wmq * current;
-      }
+    for (int m = 0; m < C; ++m) {
+      const double wmq = P.projection[static_cast<long>(m) * P.Q + node[i]];
+      acc_p[m] = acc_p[m] + wmq * pol;
+      acc_c[m] = acc_c[m] + wmq * current;
     }
   }
-  // Each wave's projections to its own rows of `red`, then the waves' sums in wave order.
+  // Each wave's projections to its own rows, then the waves' sums in wave order: the
+  // polarisation's, then the current's in the same rows (both at once would halve the
+  // workgroups a CU holds).
   const int waves = static_cast<int>(blockDim.x) / kWave;
+  wave_sync();  // the windows have been read
 #pragma unroll
-  for (int m = 0; m < C; ++m) {
-    red[(wave * 2 * C + m) * kWave + lane] = acc_p[m];
-    red[(wave * 2 * C + C + m) * kWave + lane] = acc_c[m];
+  for (int half = 0; half < 2; ++half) {
+    if (half > 0) __syncthreads();
+#pragma unroll
+    for (int m = 0; m < C; ++m) own[m * kWave + lane] = half == 0 ? acc_p[m] : acc_c[m];
+    __syncthreads();
+    if (stores)
+      for (int m = wave; m < C; m += waves) {
+        double sum = lds[m * kWave + lane];
+        for (int w = 1; w < waves; ++w) sum = sum + lds[w * ROW + m * kWave + lane];
+        B.group_streams[(static_cast<long>(group) * 2 * C + half * C + m) * T + t] = sum;
+      }
   }
-  __syncthreads();
-  if (stores)
-    for (int j = wave; j < 2 * C; j += waves) {
-      double sum = red[j * kWave + lane];
-      for (int w = 1; w < waves; ++w) sum = sum + red[(w * 2 * C + j) * kWave + lane];
-      B.group_streams[(static_cast<long>(group) * 2 * C + j) * T + t] = sum;
-    }
   if (static_cast<int>(threadIdx.x) < C) {
     const int m = threadIdx.x;
     double s = 0.0;
@@ -856,17 +925,14 @@ __device__ __forceinline__ void current_response_body(const DeviceProblem& P,
   }
 }
 
-// Five waves a SIMD up to four modes (at most 96 VGPRs): the 32 waves of each of T/63
-// tiles then take two rounds of the machine at 2^14 samples rather than three.
 template <int C>
 __global__ void __launch_bounds__(kWave * kNodeWaves)
     __attribute__((amdgpu_waves_per_eu(C <= 4 ? 5 : 4)))
     plasma_current_response(DeviceProblem P, PlasmaTable pt, const AdamsRecord* __restrict__ R,
                             FieldBuffers B) {
-  __shared__ BandLds lds;
-  __shared__ double red[kNodeWaves * 2 * C * kWave];
+  __shared__ double lds[kNodeWaves * current_lds_row<C>()];
   __shared__ double totals[kNodesPerGroup];
-  current_response_body<C>(P, pt, R, B, blockIdx.x, blockIdx.y, lds, red, totals);
+  current_response_body<C, current_lds_row<C>()>(P, pt, R, B, blockIdx.x, blockIdx.y, lds, totals);
 }
 
 // The sum of a double over the wave's 64 lanes in a fixed order, in every lane.
@@ -1599,30 +1665,22 @@ struct CorrectAt {
   }
 };
 
+// An instance with plasma runs the fused node passes (it is modal: fused_node_passes
+// holds), under either rule; one without runs the plain response alone.
 template <int C>
 struct RateAt {
-  __device__ __forceinline__ static void run(const BatchInstance& in, int tile, int group, double* table,
-                             BandLds& lds) {
-    // The fused passes read the within-tile exposure, which the band pass stores (under
-    // either rule: one tap is the trapezoid).
-    const bool fused = fused_node_passes(in.P, in.B);
-    if (in.pt.n_taps > 1 || fused)
-      rate_band_body<C>(in.P, in.pt, in.B, tile, group, table, lds, fused);
-    else
-      rate_tiles_body<C>(in.P, in.pt, in.B, tile, group, table);
+  __device__ __forceinline__ static void run(const BatchInstance& in, int tile, int group,
+                             double* lds) {
+    rate_band_body<C>(in.P, in.pt, in.B, tile, group, lds, true);
   }
 };
 
 template <int C>
 struct CurrentAt {
   __device__ __forceinline__ static void run(const BatchInstance& in, const AdamsRecord* __restrict__ R,
-                             int tile, int group, BandLds& lds, double* red, double* totals) {
-    if (fused_node_passes(in.P, in.B))
-      current_response_body<C>(in.P, in.pt, R, in.B, tile, group, lds, red, totals);
-    else if (in.pt.n_taps > 1)
-      current_band_body<C>(in.P, in.pt, R, in.B, tile, group, lds);
-    else
-      current_tiles_body<C>(in.P, R, in.B, tile, group);
+                             int tile, int group, double* lds, double* totals) {
+    current_response_body<C, current_lds_row<kMaxBatchModes>()>(in.P, in.pt, R, in.B, tile, group,
+                                                                lds, totals);
   }
 };
 
@@ -1630,10 +1688,15 @@ template <int C>
 struct ResponseAt {
   __device__ __forceinline__ static void run(const BatchInstance& in, const AdamsRecord* __restrict__ R,
                              int block, double* red) {
-    if (fused_node_passes(in.P, in.B))
-      combine_body<C>(in.P, R, in.B, block, red);
-    else
-      node_response_body<C>(in.P, R, in.B, block, red);
+    node_response_body<C>(in.P, R, in.B, block, red);
+  }
+};
+
+template <int C>
+struct CombineAt {
+  __device__ __forceinline__ static void run(const BatchInstance& in, const AdamsRecord* __restrict__ R,
+                             int block, double* offsets) {
+    combine_body<C>(in.P, R, in.B, block, offsets);
   }
 };
 
@@ -1660,31 +1723,29 @@ __global__ void __launch_bounds__(kWave) batch_predict(SP_BATCH_ARGS) {
 }
 
 __global__ void __launch_bounds__(kWave * kNodeWaves) batch_rate(SP_BATCH_ARGS) {
-  __shared__ double table[4 * kLdsTableIntervals];
-  __shared__ BandLds lds;
+  __shared__ double lds[kNodeWaves * kNodesPerWave * kWindowRow];
   const Owned o = owned(insts, records, first, n_inst);
   const BatchInstance& in = *o.inst;
   if (o.R->action == kBatchIdle) return;
   const int tiles = scan_tiles(in.P.T);
-  with_modes<RateAt>(in.P.C, in, o.local % tiles, o.local / tiles, table, lds);
+  with_modes<RateAt>(in.P.C, in, o.local % tiles, o.local / tiles, lds);
 }
 
-__global__ void __launch_bounds__(kWave) batch_prefix(SP_BATCH_ARGS, int current) {
+__global__ void __launch_bounds__(kWave) batch_prefix(SP_BATCH_ARGS) {
   const Owned o = owned(insts, records, first, n_inst);
   const BatchInstance& in = *o.inst;
   if (o.R->action == kBatchIdle) return;
-  tile_prefix_body(scan_tiles(in.P.T), current ? in.B.tile_f : in.B.tile_x, o.local);
+  tile_prefix_body(scan_tiles(in.P.T), in.B.tile_x, o.local);
 }
 
 __global__ void __launch_bounds__(kWave * kNodeWaves) batch_current(SP_BATCH_ARGS) {
-  __shared__ BandLds lds;
-  __shared__ double red[kNodeWaves * 2 * kMaxBatchModes * kWave];
+  __shared__ double lds[kNodeWaves * current_lds_row<kMaxBatchModes>()];
   __shared__ double totals[kNodesPerGroup];
   const Owned o = owned(insts, records, first, n_inst);
   const BatchInstance& in = *o.inst;
   if (o.R->action == kBatchIdle) return;
   const int tiles = scan_tiles(in.P.T);
-  with_modes<CurrentAt>(in.P.C, in, o.R, o.local % tiles, o.local / tiles, lds, red, totals);
+  with_modes<CurrentAt>(in.P.C, in, o.R, o.local % tiles, o.local / tiles, lds, totals);
 }
 
 __global__ void __launch_bounds__(kWave * kResponseWaves) batch_response(SP_BATCH_ARGS) {
@@ -1693,6 +1754,14 @@ __global__ void __launch_bounds__(kWave * kResponseWaves) batch_response(SP_BATC
   const BatchInstance& in = *o.inst;
   if (o.R->action == kBatchIdle) return;
   with_modes<ResponseAt>(in.P.C, in, o.R, o.local, red);
+}
+
+__global__ void __launch_bounds__(kWave * 4) batch_combine(SP_BATCH_ARGS) {
+  __shared__ double offsets[2 * kMaxBatchModes];
+  const Owned o = owned(insts, records, first, n_inst);
+  const BatchInstance& in = *o.inst;
+  if (o.R->action == kBatchIdle) return;
+  with_modes<CombineAt>(in.P.C, in, o.R, o.local, offsets);
 }
 
 __global__ void __launch_bounds__(kWave) batch_finish(SP_BATCH_ARGS) {
@@ -2330,18 +2399,14 @@ void launch_batch_predict(const BatchGrid& g, hipStream_t s) { grouped(batch_pre
 void launch_batch_rate(const BatchGrid& g, hipStream_t s) {
   grouped(batch_rate, g, kWave * kNodeWaves, s);
 }
-void launch_batch_prefix(const BatchGrid& g, bool current, hipStream_t s) {
-  if (g.blocks <= 0) return;
-  hipLaunchKernelGGL(batch_prefix, dim3(g.blocks), dim3(kWave), 0, s, g.inst, g.records,
-                     g.first, g.n, current ? 1 : 0);
-  SP_HIP(hipGetLastError());
-}
+void launch_batch_prefix(const BatchGrid& g, hipStream_t s) { grouped(batch_prefix, g, kWave, s); }
 void launch_batch_current(const BatchGrid& g, hipStream_t s) {
   grouped(batch_current, g, kWave * kNodeWaves, s);
 }
 void launch_batch_response(const BatchGrid& g, hipStream_t s) {
   grouped(batch_response, g, kWave * kResponseWaves, s);
 }
+void launch_batch_combine(const BatchGrid& g, hipStream_t s) { grouped(batch_combine, g, kWave * 4, s); }
 void launch_batch_finish(const BatchGrid& g, hipStream_t s) { grouped(batch_finish, g, kWave, s); }
 void launch_batch_correct(const BatchGrid& g, hipStream_t s) { grouped(batch_correct, g, kWave, s); }
 void launch_batch_norms(const BatchGrid& g, hipStream_t s) { grouped(batch_norms, g, kNormThreads, s); }

@@ -159,8 +159,9 @@ struct BatchGrid {
 void launch_batch_commit(const BatchGrid& g, hipStream_t s);
 void launch_batch_predict(const BatchGrid& g, hipStream_t s);
 void launch_batch_rate(const BatchGrid& g, hipStream_t s);
-void launch_batch_prefix(const BatchGrid& g, bool current, hipStream_t s);
+void launch_batch_prefix(const BatchGrid& g, hipStream_t s);
 void launch_batch_current(const BatchGrid& g, hipStream_t s);
+void launch_batch_combine(const BatchGrid& g, hipStream_t s);
 void launch_batch_response(const BatchGrid& g, hipStream_t s);
 void launch_batch_finish(const BatchGrid& g, hipStream_t s);
 void launch_batch_correct(const BatchGrid& g, hipStream_t s);

@@ -176,7 +176,6 @@ void Scan::plan_launches() {
   inst_dev_ = device_upload(allocations_, host.data(), host.size());
 
   std::vector<int> first;
-  std::vector<char> fused(static_cast<std::size_t>(n), 0);
   auto table = [&](Group& g, auto blocks_of) {
     g.offset = static_cast<int>(first.size());
     int total = 0;
@@ -197,15 +196,13 @@ void Scan::plan_launches() {
   table(rate_, node_blocks);
   table(current_, node_blocks);
   table(prefix_, [&](const DeviceProblem& P) { return P.has_plasma ? P.Q : 0; });
-  for (int i = 0; i < n; ++i) fused[i] = fused_node_passes(host[i].P, host[i].B);
-  int at = 0;
-  table(prefix_current_, [&](const DeviceProblem& P) {
-    return P.has_plasma && !fused[at++] ? P.Q : 0;
-  });
-  table(response_, [&](const DeviceProblem& P) {
-    SP_CHECK(P.T % kWave == 0, "the node response takes 64-sample blocks");
-    return P.T / kWave;
-  });
+  for (int i = 0; i < n; ++i) {
+    SP_CHECK(host[i].P.T % kWave == 0, "the node response takes 64-sample blocks");
+    SP_CHECK(!host[i].P.has_plasma || fused_node_passes(host[i].P, host[i].B),
+             "a scan instance with plasma runs the fused node passes");
+  }
+  table(combine_, [&](const DeviceProblem& P) { return P.has_plasma ? P.T / kWave : 0; });
+  table(response_, [&](const DeviceProblem& P) { return P.has_plasma ? 0 : P.T / kWave; });
   table(finish_, [&](const DeviceProblem& P) {
     return static_cast<int>(blocks_for(static_cast<std::size_t>(P.C) * (P.T / 4 + 1), kWave));
   });
@@ -386,9 +383,9 @@ void Scan::enqueue_round() {
   for (const FftGroup& g : inverse_)
     launch_fft_grouped(g.log2L, g.log2G, g.jobs, g.first, g.n, g.blocks, +1, stream_);
   launch_batch_rate(grid(rate_), stream_);
-  launch_batch_prefix(grid(prefix_), false, stream_);
+  launch_batch_prefix(grid(prefix_), stream_);
   launch_batch_current(grid(current_), stream_);
-  launch_batch_prefix(grid(prefix_current_), true, stream_);
+  launch_batch_combine(grid(combine_), stream_);
   launch_batch_response(grid(response_), stream_);
   for (const FftGroup& g : forward_)
     launch_fft_grouped(g.log2L, g.log2G, g.jobs, g.first, g.n, g.blocks, -1, stream_);
