@@ -79,8 +79,10 @@ class FftPlan {
   FftPlan(const FftPlan&) = delete;
   FftPlan& operator=(const FftPlan&) = delete;
 
-  // A complex transform of n points over `batch` contiguous rows of n.
-  void init(std::size_t n, std::size_t batch);
+  // A complex transform of n points over `batch` contiguous rows of n. With `few_rows` a
+  // transform that one pass could hold is split in two all the same where its rows would
+  // leave the chip idle (layout); exec then needs its scratch.
+  void init(std::size_t n, std::size_t batch, bool few_rows = false);
   // The same plan with its twiddle tables in device memory the caller owns, at least
   // table_points(n) points at `tables`: nothing is allocated or freed. The tables hold
   // nothing until upload_tables has run (on `stream`, which it then synchronises).
@@ -109,7 +111,7 @@ class FftPlan {
   std::size_t bytes() const { return bytes_; }
 
  private:
-  void layout(std::size_t n, std::size_t batch);
+  void layout(std::size_t n, std::size_t batch, bool few_rows = false);
   void launch(const FftPass& p, const cplx* in, cplx* out, int sign, hipStream_t s) const;
   std::size_t n_ = 0, batch_ = 0, bytes_ = 0;
   bool owns_tables_ = true;

@@ -244,8 +244,8 @@ void FieldWorkspace::allocate(const sp_problem_desc& d) {
   // row it transforms.
   const std::size_t forward_rows = ((d.has_plasma ? 3 : 1) + (absorbing() ? 1 : 0)) * C;
   scratch_ = alloc<cplx>((forward_rows > 3UL * C ? forward_rows : 3UL * C) * (T / 2));
-  inv_plan_.init(T / 2, C);
-  fwd_plan_.init(T / 2, forward_rows);
+  inv_plan_.init(T / 2, C, true);
+  fwd_plan_.init(T / 2, forward_rows, true);
   if (d.n_raman) {
     // The doubled-grid drive of every node, its transform scratch, the kernel's packed
     // samples and spectrum, and the roots of 2T for the real-transform packing.
