@@ -81,6 +81,11 @@ enum Status : int {
     if (!(cond)) throw ::sp::Error(::sp::kValue, (msg));     \
   } while (0)
 
+// Stores a sum that the host awaits by its value (sync.hpp).
+__device__ inline void store_awaited(double* at, double value) {
+  __hip_atomic_store(at, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The owner of workgroup `block` in a grouped launch whose owners hold consecutive ranges:
 // owner i holds first[i] .. first[i + 1] - 1 (first[0] = 0, first[n] = the grid). A binary
 // search, the same in every lane of the workgroup.

@@ -370,7 +370,8 @@ __global__ void __launch_bounds__((EnvShape<LOG2L, Kind>::THREADS))
           for (int i = 0; i < 3; ++i) sums[i][tid] = sums[i][tid] + sums[i][tid + half];
         __syncthreads();
       }
-      if (tid < 3) a.partials[tid * static_cast<int>(gridDim.x) + blockIdx.x] = sums[tid][0];
+      if (tid < 3)
+        store_awaited(a.partials + tid * static_cast<int>(gridDim.x) + blockIdx.x, sums[tid][0]);
     } else {
       __syncthreads();
       F::inputs(u, [&](cplx& x, int s, int k) { x = lds[k * G + s]; });

@@ -1551,7 +1551,7 @@ __device__ __forceinline__ void norms_body(const double* __restrict__ partials, 
     if (j < half) tree[threadIdx.x] = tree[threadIdx.x] + tree[threadIdx.x + half];
     __syncthreads();
   }
-  if (j == 0) norms[s] = tree[threadIdx.x];
+  if (j == 0) store_awaited(norms + s, tree[threadIdx.x]);
 }
 
 __global__ void __launch_bounds__(kNormThreads)
@@ -1898,7 +1898,7 @@ __global__ void __launch_bounds__(kLsThreads)
       if (threadIdx.x < half) tree[threadIdx.x] = tree[threadIdx.x] + tree[threadIdx.x + half];
       __syncthreads();
     }
-    if (threadIdx.x == 0) norms[k] = tree[0];
+    if (threadIdx.x == 0) store_awaited(norms + k, tree[0]);
     __syncthreads();
   }
 }

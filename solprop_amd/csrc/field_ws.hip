@@ -278,7 +278,6 @@ void FieldWorkspace::allocate(const sp_problem_desc& d) {
     ls_partials_ = alloc<double>(ls_partials(ls_blocks(P_)));
   }
   for (hipEvent_t& e : marks_) SP_HIP(hipEventCreate(&e));
-  SP_HIP(hipEventCreateWithFlags(&done_, hipEventDisableTiming));
   slot_rates_.assign(S, std::vector<double>(kMaxTerms, 0.0));
   if (d.n_raman && !raman_dynamic_) {
     // Constant rates: the kernel's spectrum once, here.
@@ -306,8 +305,6 @@ void FieldWorkspace::release() {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
   }
-  if (done_) (void)hipEventDestroy(done_);
-  done_ = nullptr;
   if (stream_ && own_stream_) (void)hipStreamDestroy(stream_);
   graphs_.clear();
   allocations_.clear();
@@ -467,14 +464,6 @@ void FieldWorkspace::run(int key) {
   }
   SP_HIP(hipGraphLaunch(it->second, stream_));
   graph_launches_ += 1;
-}
-
-void FieldWorkspace::wait() {
-  // Poll the stream's last event: the host's next decision needs this trial's sums as
-  // soon as they land (a blocking wait adds a wake-up); past a short spin the poll
-  // yields and backs off, and a device that never finishes is reported.
-  SP_HIP(hipEventRecord(done_, stream_));
-  wait_event(done_);
 }
 
 void FieldWorkspace::flush() {
@@ -642,12 +631,13 @@ std::vector<double> FieldWorkspace::trial(double z, double dz, const adams::Sten
   // The trial's source evaluation replaces B.lab: the last accepted one's is gone.
   quad_ready_ = false;
   trial_end_ = z + dz;
+  expect_sums(norms_host_, 1 + kMaxScored);
   run((pending_slot_ >= 0 ? kCommitTrial : kTrial) + 16 * width_);
   pending_slot_ = -1;
   if (marking_)
     SP_HIP(hipStreamSynchronize(stream_));
   else
-    wait();
+    wait_sums(norms_host_, 1 + kMaxScored, stream_);
   if (marking_) {
     float ms = 0.0f;
     for (int i = 0; i < kPhases; ++i) {
@@ -708,6 +698,7 @@ double FieldWorkspace::ls_trial(double z, double dz) {
     ls_rec_host_[1].x_w[t] = path_increment(phi_paths_[t], mid, end);
   }
   marking_ = false;
+  expect_sums(norms_host_, 3);
   if (use_graphs_) {
     if (!ls_graph_) ls_graph_ = capture_graph(stream_, [&] { enqueue_ls_step(); });
     SP_HIP(hipGraphLaunch(ls_graph_, stream_));
@@ -715,7 +706,7 @@ double FieldWorkspace::ls_trial(double z, double dz) {
   } else {
     enqueue_ls_step();
   }
-  wait();
+  wait_sums(norms_host_, 3, stream_);
   trials_ += 1;
   evaluations_ += 4;
   const double lower = std::sqrt(norms_host_[0]), upper = std::sqrt(norms_host_[1]);

@@ -214,7 +214,6 @@ Workspace::Workspace(const sp_problem_desc& d) {
   SP_HIP(hipHostMalloc(reinterpret_cast<void**>(&partials_host_),
                        3 * sizeof(double) * n_partial_blocks_, hipHostMallocMapped));
   SP_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&env_.partials), partials_host_, 0));
-  SP_HIP(hipEventCreateWithFlags(&done_, hipEventDisableTiming));
   SP_HIP(hipEventCreate(&ev0_));
   SP_HIP(hipEventCreate(&ev1_));
 }
@@ -225,7 +224,6 @@ Workspace::~Workspace() {
   for (void* p : allocations_) (void)hipFree(p);
   if (rec_host_) (void)hipHostFree(rec_host_);
   if (partials_host_) (void)hipHostFree(partials_host_);
-  if (done_) (void)hipEventDestroy(done_);
   if (ev0_) (void)hipEventDestroy(ev0_);
   if (ev1_) (void)hipEventDestroy(ev1_);
   if (stream_) (void)hipStreamDestroy(stream_);
@@ -315,9 +313,9 @@ void Workspace::enqueue_trial(bool commit, Stage0 mode) {
 
 double Workspace::finish_trial() {
   if (profile_) SP_HIP(hipEventRecord(ev1_, stream_));
-  SP_HIP(hipEventRecord(done_, stream_));
-  wait_event(done_);
+  wait_sums(partials_host_, 3 * n_partial_blocks_, stream_);
   if (profile_) {
+    SP_HIP(hipEventSynchronize(ev1_));
     float ms = 0.0f;
     SP_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
     time_total_ms_ += ms;
@@ -348,6 +346,7 @@ double Workspace::trial(double z, double dz, bool full) {
       mode = kKeep;
   }
   if (profile_) SP_HIP(hipEventRecord(ev0_, stream_));
+  expect_sums(partials_host_, 3 * n_partial_blocks_);
   const int key = (commit ? 4 : 0) + static_cast<int>(mode);
   if (use_graphs_) {
     auto it = graphs_.find(key);

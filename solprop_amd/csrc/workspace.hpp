@@ -101,7 +101,7 @@ class Workspace final : public Propagator {
   // Counters and timing.
   long trials_ = 0, evaluations_ = 0, accepted_ = 0, graph_launches_ = 0;
   bool profile_ = false;
-  hipEvent_t ev0_ = nullptr, ev1_ = nullptr, done_ = nullptr;
+  hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
   double time_total_ms_ = 0.0;
   long timed_ = 0;
 };
