@@ -451,6 +451,63 @@ __device__ inline void band_filter_nodes(const PlasmaTable& pt, const double* wi
       f[i] = f[i] + pt.taps[k] * (y[i * kWindowRow - k] + y[i * kWindowRow + k]);
 }
 
+// Which of N nodes extra sample `idx` belongs to, S a node (a division would take longer
+// than the sample).
+template <int N>
+__device__ inline int extra_node(int idx, int S) {
+  int i = 0;
+#pragma unroll
+  for (int k = 1; k < N; ++k) i += idx >= k * S ? 1 : 0;
+  return i;
+}
+
+// The fraction at an exposure of zero: fraction_of with its exponential one.
+__device__ inline double fraction_at_rest(double f0) {
+#pragma clang fp contract(off)
+  return 1.0 - (1.0 - f0) * 1.0;
+}
+
+// `v` of one lane, in every lane.
+__device__ inline double from_lane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// The fractions of a wave's nodes at the lanes' exposures. Most tiles lie away from the
+// pulse: where nothing has been exposed the exponential is one, and where every lane but
+// the last (the next tile's first sample) holds its tile's offset, `level`, two lanes a
+// node evaluate it for all: one exponential instead of N. The same values.
+template <int N>
+__device__ inline void fractions(double f0, const double (&x)[N], bool level, int lane,
+                                 double (&f)[N]) {
+  bool exposed = false;
+#pragma unroll
+  for (int i = 0; i < N; ++i) exposed = exposed || x[i] > 0.0;
+  if (__ballot(exposed) == 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) f[i] = fraction_at_rest(f0);
+    return;
+  }
+  if (level) {
+    double mine = 0.0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const double first = from_lane(x[i], 0), last = from_lane(x[i], kWave - 1);
+      if (lane == i) mine = first;
+      if (lane == N + i) mine = last;
+    }
+    const double v = fraction_of(f0, mine > 0.0 ? mine : 0.0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const double first = from_lane(v, i), last = from_lane(v, N + i);
+      f[i] = lane == kWave - 1 ? last : first;
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) f[i] = fraction_of(f0, x[i] > 0.0 ? x[i] : 0.0);
+}
+
 template <int Ctrl, int RowMask, bool Bound, int N>
 __device__ inline void scan_step(double (&v)[N]) {
 #pragma unroll
@@ -502,7 +559,8 @@ __device__ inline double current_sample_sparse(const DeviceProblem& P, const Fie
   const long at = static_cast<long>(q) * tiles + owner;
   const double* local = B.zero_tiles[at] ? &kZeroSample : B.x_local + static_cast<long>(q) * P.T + t;
   const double x = B.tile_x[at] + *local;
-  const double f = fraction_of(f0, x > 0.0 ? x : 0.0);
+  double f = fraction_at_rest(f0);
+  if (x > 0.0) f = fraction_of(f0, x);
   double am[held(C)];
   load_modal<C>(B, P.T, t, am);
   return (f * P.plasma_cmr) * field_at<C>(P, B, am, q, t);
@@ -600,7 +658,7 @@ __device__ __forceinline__ void rate_band_body(const DeviceProblem& P, const Pla
   load_modal<C>(B, T, tc, am);
   const bool inner = tile * kTileSpan >= K && tile * kTileSpan + kWave - 1 + K <= T - 1;
   for (int idx = lane; idx < NPW * S; idx += kWave) {
-    const int i = idx / S, h = idx - i * S;
+    const int i = extra_node<NPW>(idx, S), h = idx - i * S;
     const int q = min(q0 + i * kNodeWaves, P.Q - 1);
     auto sample = [&](int u) { return rate_sample<C>(P, pt, coefficients, B, q, u); };
     const int u = extra_sample(tile, K, T, h);
@@ -827,7 +885,7 @@ __device__ __forceinline__ void current_response_body(const DeviceProblem& P,
   bool busy = false;
   const bool inner = tile * kTileSpan >= K && tile * kTileSpan + kWave - 1 + K <= T - 1;
   for (int idx = lane; idx < NPW * S; idx += kWave) {
-    const int i = idx / S, h = idx - i * S;
+    const int i = extra_node<NPW>(idx, S), h = idx - i * S;
     const int q = min(q0 + i * kNodeWaves, P.Q - 1);
     auto sample = [&](int u) { return current_sample_sparse<C>(P, B, q, u, f0, tiles); };
     const int u = extra_sample(tile, K, T, h);
@@ -836,9 +894,12 @@ __device__ __forceinline__ void current_response_body(const DeviceProblem& P,
     own[i * kWindowRow + (h < H ? halo_slot(K, h) : kBandSpan + h - H)] = v;
   }
   double f[NPW], e[NPW], y[NPW];
+  bool flagged = t < T;
+#pragma unroll
+  for (int i = 0; i < NPW; ++i) flagged = flagged && zero[i];
+  fractions<NPW>(f0, xs, __ballot(flagged) == ~0ULL, lane, f);
 #pragma unroll
   for (int i = 0; i < NPW; ++i) {
-    f[i] = fraction_of(f0, xs[i] > 0.0 ? xs[i] : 0.0);
     e[i] = synthesise_at<C>(P.synthesis + static_cast<long>(node[i]) * C, am);
     y[i] = (f[i] * P.plasma_cmr) * e[i];
   }
