@@ -70,7 +70,9 @@ __device__ inline float sum16(float v) {
   return v;
 }
 
-// A lane's eight spectral elements of one channel from the (MP, rows, WP) layout.
+// A lane's eight spectral elements of one channel from the (MP, rows, WP) layout. (Eight
+// together in a (rows, WP, MP) layout gain the layers nothing and cost the mixing's stores
+// half its time again.)
 __device__ inline v8b load_spectrum(const bf16* y, int k0, int b, int c, int rows, int WP) {
   us8 v;
 #pragma unroll
@@ -321,11 +323,28 @@ __global__ void __launch_bounds__(256) tile_mix(MixArgs a) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
   const int k = blockIdx.x, b0 = blockIdx.y * 16;
   const long plane = static_cast<long>(MP) * a.B * WP;
+  // The wave's weights first, all at once: they wait for nothing, and the shares' loads
+  // (eight in flight, added in order) overlap theirs. Loaded between the products they were
+  // most of the kernel's 12.1 us at 64 channels and samples; now 6.5 us.
+  const int o = 16 * wave + l16;
+  float wr[WP / 4], wi[WP / 4];
+  if (wave < WP / 16) {
+#pragma unroll
+    for (int n = 0; n < WP / 4; ++n) {
+      const int i = 16 * (n / 4) + 4 * q + n % 4;
+      const bool have = i < a.W && o < a.W;
+      const long at = BACK ? (static_cast<long>(k) * a.W + o) * a.W + i
+                           : (static_cast<long>(k) * a.W + i) * a.W + o;
+      wr[n] = have ? a.rre[at] : 0.f;
+      wi[n] = have ? a.rim[at] : 0.f;
+    }
+  }
   for (int e = tid; e < 2 * 16 * WP / 4; e += 256) {
     const int part = e / (16 * WP / 4), row = e / (WP / 4) % 16, c = e % (WP / 4) * 4;
     v4f v = {0.f, 0.f, 0.f, 0.f};
     if (b0 + row < a.B) {
       const long at = (static_cast<long>(k + part * (MP / 2)) * a.B + b0 + row) * WP + c;
+#pragma unroll 8
       for (int z = 0; z < a.chunks; ++z)
         v += *reinterpret_cast<const v4f*>(a.share + z * plane + at);
       if (a.total) *reinterpret_cast<v4f*>(a.total + at) = v;
@@ -334,7 +353,6 @@ __global__ void __launch_bounds__(256) tile_mix(MixArgs a) {
   }
   __syncthreads();
   if (wave >= WP / 16) return;
-  const int o = 16 * wave + l16;
   v4f yr = {0.f, 0.f, 0.f, 0.f}, yi = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int t = 0; t < WP / 16; ++t) {
@@ -342,11 +360,7 @@ __global__ void __launch_bounds__(256) tile_mix(MixArgs a) {
     const v4f vi = *reinterpret_cast<const v4f*>(&in[1][l16 * kCol + 16 * t + 4 * q]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = 16 * t + 4 * q + r;
-      const bool have = i < a.W && o < a.W;
-      const long at = BACK ? (static_cast<long>(k) * a.W + o) * a.W + i
-                           : (static_cast<long>(k) * a.W + i) * a.W + o;
-      const float rr = have ? a.rre[at] : 0.f, ri = have ? a.rim[at] : 0.f;
+      const float rr = wr[4 * t + r], ri = wi[4 * t + r];
       yr = mfma32(vr[r], rr, yr);
       yi = mfma32(vi[r], rr, yi);
       yr = mfma32(BACK ? vi[r] : -vi[r], ri, yr);
