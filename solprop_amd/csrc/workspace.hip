@@ -417,6 +417,7 @@ void Workspace::load(double z, const double* field) {
 void Workspace::read_state(double* out) {
   if (!loaded_) throw Error(kState, "no state is loaded");
   ensure_committed();
+  SP_HIP(hipStreamSynchronize(stream_));  // a trial's last kernel may still be ending
   SP_HIP(hipMemcpy(out, y_, sizeof(cplx) * P_.C * P_.N, hipMemcpyDeviceToHost));
 }
 
