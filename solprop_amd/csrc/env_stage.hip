@@ -121,20 +121,39 @@ __device__ inline cplx bin_derivative(const EnvStage& a, const BinFinish& f, int
 // chip is full all the same, and neighbouring sequences share the lines that a stored or
 // gathered point would touch alone. A march of 20 attempts on 2^15 samples takes 3.23 ms
 // at 2^9 points, 3.61 at 2^8 and 3.39 at 2^10; a trial on 2^17, 506, 567 and 473 us.
+// Sequences of 1024 points or more (2^19 samples on) take 2^12 points, what LDS holds: a
+// lone sequence moved a line for every point it stored or gathered. A trial on 2^20 bins
+// took 1.83 ms; in the order of sequence_group 0.91 at 2^10 points, 0.65 at 2^11 and 0.55
+// at 2^12 (1.32 with the transforms and the work at the bins apart).
 constexpr int env_log2g(int log2l, bool bins) {
-  const int want = (log2l >= (bins ? 8 : 9) ? 10 : 9) - log2l, most = log2l > 1 ? log2l - 1 : 0;
+  const int points = log2l >= 10 ? 12 : (log2l >= (bins ? 8 : 9) ? 10 : 9);
+  const int want = points - log2l, most = log2l > 1 ? log2l - 1 : 0;
   const int g = want < 0 ? 0 : want;
   return g < most ? g : most;
 }
 
+// The group of sequences a workgroup takes. Workgroups go to the eight XCDs in turn; each
+// XCD takes a consecutive run of groups, so that the workgroups that share a line share an
+// L2 (in launch order every XCD fetched, and wrote in parts, every line of the strided
+// side). For sequences of 256 points or more, whose launches hold a multiple of 32 groups:
+// below, a launch is too short for it (2^14 samples 93 us either way). A trial on 2^16 bins
+// and samples 133 -> 112 us, on 2^19 610 -> 366.
+template <int LOG2L>
+__device__ inline int sequence_group() {
+  const int b = static_cast<int>(blockIdx.x), n = static_cast<int>(gridDim.x);
+  return LOG2L >= 8 ? b % 8 * (n / 8) + b / 8 : b;
+}
+
 // The kernels with work at the bins (two exponentials and a sine and cosine each) take a
-// thread a point, the others a thread eight points.
+// thread a point (one to four on the long sequences), the others a thread eight points.
 template <int LOG2L, int Kind>
 struct EnvShape {
   static constexpr int L = 1 << LOG2L;
   static constexpr bool bins = Kind == kEntry || Kind == kFinish || Kind == kAccept;
   static constexpr int G = 1 << env_log2g(LOG2L, bins);
   static constexpr int E = L * G;
+  // A long strided side moves whole lines, 64 bytes, unless LDS holds no more sequences.
+  static_assert(LOG2L < 10 || G >= 4 || E == 4096);
   static constexpr int THREADS = bins ? (E < 1024 ? E : 1024) : (E >= 8 ? E / 8 : 1);
   static constexpr bool held = LOG2L <= 9 && THREADS <= 512;  // twiddles in registers
   using First = RegsFft<LOG2L, G, true, false, 3, THREADS>;
@@ -153,7 +172,8 @@ __global__ void __launch_bounds__((EnvShape<LOG2L, Kind>::THREADS))
   constexpr int POINTS = (E + NT - 1) / NT;  // points a thread takes at the bins
   const DeviceProblem& P = a.P;
   const int tid = threadIdx.x;
-  const int s0 = static_cast<int>(blockIdx.x) * G;
+  const int group = sequence_group<LOG2L>();
+  const int s0 = group * G;
   const int S = P.T >> LOG2L;
   const cplx* tw = a.roots_l[LOG2L == a.log2n1 ? 0 : 1];
   __shared__ cplx lds[E];
@@ -371,7 +391,7 @@ __global__ void __launch_bounds__((EnvShape<LOG2L, Kind>::THREADS))
         __syncthreads();
       }
       if (tid < 3)
-        store_awaited(a.partials + tid * static_cast<int>(gridDim.x) + blockIdx.x, sums[tid][0]);
+        store_awaited(a.partials + tid * static_cast<int>(gridDim.x) + group, sums[tid][0]);
     } else {
       __syncthreads();
       F::inputs(u, [&](cplx& x, int s, int k) { x = lds[k * G + s]; });
@@ -404,6 +424,7 @@ template <int LOG2L, int Kind>
 void launch_kind(const EnvStage& a, int stage, hipStream_t s) {
   using H = EnvShape<LOG2L, Kind>;
   const unsigned blocks = static_cast<unsigned>((a.P.T >> LOG2L) / H::G);
+  SP_CHECK(LOG2L < 8 || blocks % 8 == 0, "the groups of long sequences run in eights");
   hipLaunchKernelGGL((env_kernel<LOG2L, Kind>), dim3(blocks), dim3(H::THREADS), 0, s, a, stage);
 }
 

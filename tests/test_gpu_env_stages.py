@@ -12,7 +12,7 @@ import pytest
 from test_gpu_rk import norm_bound, oracle_trial, rel_l2
 
 from solprop_amd.native import Workspace
-from solprop_amd.problem import ScalarPath, gnlse_problem
+from solprop_amd.problem import ScalarPath, Tableau, gnlse_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -50,6 +50,29 @@ def test_trial_over_the_splits(n_t, ffac, option):
         size = np.abs(problem.field0).max() or 1.0
         problem.field0 = size * problem.active_mask * np.exp(
             2j * np.pi * rng.uniform(size=problem.field0.shape))
+    dz = 1e-4
+    advanced, norm, _ = oracle_trial(problem, dz)
+    ws = Workspace(problem)
+    probe = ws.probe(0.0, problem.field0)
+    got = probe.trial(0.0, dz)
+    field = probe.field()
+    ws.close()
+    assert rel_l2(field, advanced.reshape(field.shape)) < 1e-12
+    y0 = problem.field0.reshape(field.shape)
+    assert abs(got - norm) <= norm_bound(problem, advanced, y0)
+
+
+# From 2^20 samples the kernels at the bins take two to four points a thread; 2^22 to 2^24
+# split in sequences of 2048 and 4096 points, the longest. Two stages (Heun's pair) run
+# every kernel and keep the oracle's time to seconds.
+@pytest.mark.parametrize("n_t, ffac, option", [
+    (2**20, 1, "absorber_noise"), (2**20, 4, "absorber_noise"), (2**20, 8, "raman"),
+    (2**20, 16, "absorber_noise")])
+def test_longest_sequences(n_t, ffac, option):
+    print("envelope trial, two stages", n_t, ffac, option, flush=True)
+    problem = problem_of(n_t, ffac, option)
+    problem.tableau = Tableau(np.array([0.0, 1.0]), np.array([[0.0, 0.0], [1.0, 0.0]]),
+                              np.array([0.5, 0.5]), np.array([-0.5, 0.5]), False)
     dz = 1e-4
     advanced, norm, _ = oracle_trial(problem, dz)
     ws = Workspace(problem)
