@@ -31,11 +31,16 @@ __device__ inline cplx kerr_point(cplx e, const KerrArgs& k) {
 // 256 x 128 x 512 points (268 MB a pass either way), before with radix-4 stages in LDS and
 // now: x pass 158 -> 84 us (6.4 TB/s), y response 140 -> 98 us.
 
+// A thread of a strided pass holds a radix-16 butterfly, or a whole sequence where that is
+// shorter.
+template <int LOG2L, int G, bool RestFirst>
+using AxisFft = RegsFft<LOG2L, G, true, RestFirst, (LOG2L < 4 ? LOG2L : 4)>;
+
 // The x axis: G neighbouring sequences (points `stride` apart, blocks of L stride points).
 template <int LOG2L, int G, int Sign>
-__global__ void __launch_bounds__((RegsFft<LOG2L, G, true, false>::NT))
+__global__ void __launch_bounds__((AxisFft<LOG2L, G, false>::NT))
     cart_x(cplx* f, long stride, const cplx* __restrict__ tw) {
-  using F = RegsFft<LOG2L, G, true, false>;
+  using F = AxisFft<LOG2L, G, false>;
   __shared__ cplx lds[F::LDS_POINTS];
   cplx* at = f + static_cast<long>(blockIdx.y) * F::L * stride + static_cast<long>(blockIdx.x) * G;
   typename F::First v;
@@ -49,10 +54,10 @@ __global__ void __launch_bounds__((RegsFft<LOG2L, G, true, false>::NT))
 // in one pass, in place: the forward transform's stages run in the reverse order of
 // radices, so that it starts from the registers the inverse ends with.
 template <int LOG2L, int G>
-__global__ void __launch_bounds__((RegsFft<LOG2L, G, true, false>::NT))
+__global__ void __launch_bounds__((AxisFft<LOG2L, G, false>::NT))
     cart_y_response(cplx* f, long stride, const cplx* __restrict__ tw, KerrArgs k) {
-  using I = RegsFft<LOG2L, G, true, false>;
-  using F = RegsFft<LOG2L, G, true, true>;
+  using I = AxisFft<LOG2L, G, false>;
+  using F = AxisFft<LOG2L, G, true>;
   __shared__ cplx lds[I::LDS_POINTS];
   cplx* at = f + static_cast<long>(blockIdx.x) * G;
   typename I::First v;
@@ -124,10 +129,10 @@ __device__ inline cplx table_flow(const void* table, long idx, double w) {
   }
 }
 
-template <int LOG2L, int G, int Kind, bool Imaginary>
-__global__ void __launch_bounds__((RegsFft<LOG2L, G, false, false>::NT))
+template <int LOG2L, int G, int LOGR, int Kind, bool Imaginary>
+__global__ void __launch_bounds__((RegsFft<LOG2L, G, false, false, LOGR>::NT))
     cart_t(TArgs a, const cplx* __restrict__ tw) {
-  using F = RegsFft<LOG2L, G, false, false>;
+  using F = RegsFft<LOG2L, G, false, false, LOGR>;
   constexpr int L = F::L, E = F::E, NT = F::NT;
   __shared__ cplx lds[F::LDS_POINTS];
   __shared__ double tree[NT];
@@ -222,7 +227,7 @@ __global__ void take_imaginary(const cplx* __restrict__ table, std::size_t n,
 template <int LOG2L, int G>
 struct XPass {
   static void launch(dim3 grid, hipStream_t s, cplx* f, long stride, const cplx* tw, int sign) {
-    constexpr int NT = RegsFft<LOG2L, G, true, false>::NT;
+    constexpr int NT = AxisFft<LOG2L, G, false>::NT;
     if (sign > 0)
       hipLaunchKernelGGL((cart_x<LOG2L, G, 1>), grid, dim3(NT), 0, s, f, stride, tw);
     else
@@ -235,38 +240,41 @@ struct YResponse {
   static void launch(unsigned blocks, hipStream_t s, cplx* f, long stride, const cplx* tw,
                      KerrArgs k) {
     hipLaunchKernelGGL((cart_y_response<LOG2L, G>), dim3(blocks),
-                       dim3(RegsFft<LOG2L, G, true, false>::NT), 0, s, f, stride, tw, k);
+                       dim3(AxisFft<LOG2L, G, false>::NT), 0, s, f, stride, tw, k);
   }
 };
 
-template <int LOG2L, int G>
+template <int LOG2L, int G, int LOGR>
 struct TStage {
   template <bool Imaginary>
   static void launch(int kind, unsigned blocks, hipStream_t s, const TArgs& a, const cplx* tw) {
-    const dim3 grid(blocks), block(RegsFft<LOG2L, G, false, false>::NT);
+    const dim3 grid(blocks), block(RegsFft<LOG2L, G, false, false, LOGR>::NT);
     switch (kind) {
       case kInverse:  // reads neither table
-        hipLaunchKernelGGL((cart_t<LOG2L, G, kInverse, true>), grid, block, 0, s, a, tw);
+        hipLaunchKernelGGL((cart_t<LOG2L, G, LOGR, kInverse, true>), grid, block, 0, s, a, tw);
         break;
       case kPass1:
-        hipLaunchKernelGGL((cart_t<LOG2L, G, kPass1, Imaginary>), grid, block, 0, s, a, tw);
+        hipLaunchKernelGGL((cart_t<LOG2L, G, LOGR, kPass1, Imaginary>), grid, block, 0, s, a, tw);
         break;
       case kPass2:
-        hipLaunchKernelGGL((cart_t<LOG2L, G, kPass2, Imaginary>), grid, block, 0, s, a, tw);
+        hipLaunchKernelGGL((cart_t<LOG2L, G, LOGR, kPass2, Imaginary>), grid, block, 0, s, a, tw);
         break;
       case kPass3:
-        hipLaunchKernelGGL((cart_t<LOG2L, G, kPass3, Imaginary>), grid, block, 0, s, a, tw);
+        hipLaunchKernelGGL((cart_t<LOG2L, G, LOGR, kPass3, Imaginary>), grid, block, 0, s, a, tw);
         break;
       case kPass4:
-        hipLaunchKernelGGL((cart_t<LOG2L, G, kPass4, Imaginary>), grid, block, 0, s, a, tw);
+        hipLaunchKernelGGL((cart_t<LOG2L, G, LOGR, kPass4, Imaginary>), grid, block, 0, s, a, tw);
         break;
       default:
-        hipLaunchKernelGGL((cart_t<LOG2L, G, kSource, Imaginary>), grid, block, 0, s, a, tw);
+        hipLaunchKernelGGL((cart_t<LOG2L, G, LOGR, kSource, Imaginary>), grid, block, 0, s, a, tw);
     }
   }
 };
 
-// The strided passes' shapes: workgroups of at most kMaxElems points.
+// The strided passes' shapes: workgroups of at most kMaxElems points, 16 sequences or, on an
+// axis of at most kShortAxis points, 64 (a thread each).
+constexpr int kShortAxis = 8;
+
 template <template <int, int> class Op, int LOG2L, typename... A>
 void dispatch_g(int log2g, A... a) {
   constexpr int L = 1 << LOG2L;
@@ -276,6 +284,8 @@ void dispatch_g(int log2g, A... a) {
     case 2: if constexpr (L * 4 <= kMaxElems) { Op<LOG2L, 4>::launch(a...); return; } break;
     case 3: if constexpr (L * 8 <= kMaxElems) { Op<LOG2L, 8>::launch(a...); return; } break;
     case 4: if constexpr (L * 16 <= kMaxElems) { Op<LOG2L, 16>::launch(a...); return; } break;
+    case 5: if constexpr (L <= kShortAxis) { Op<LOG2L, 32>::launch(a...); return; } break;
+    case 6: if constexpr (L <= kShortAxis) { Op<LOG2L, 64>::launch(a...); return; } break;
     default: break;
   }
   throw Error(kValue, "no Cartesian pass kernel for this shape");
@@ -300,28 +310,40 @@ void dispatch(int log2l, int log2g, A... a) {
   SP_HIP(hipGetLastError());
 }
 
-// The t rows a workgroup owns (log2): enough for 2^10 points (one wave, so that its
-// barriers wait for nobody: stage 1 344 -> 325 us and stage 4 265 -> 242 us against 2^11
-// points on 512-point rows), or 2^8 where that would leave fewer than 256 workgroups; at
-// most 16 rows, which divide any grid's nx ny.
+// The t rows a workgroup owns (log2): enough for 2^10 points (one wave of 16 points a
+// thread, so that its barriers wait for nobody: stage 1 344 -> 325 us and stage 4 265 ->
+// 242 us against 2^11 points on 512-point rows). Where that leaves fewer than 1024
+// workgroups the chip is not full and a step waits for one thread's chain of points: then
+// 2^8 points and four a thread (16 a thread are a quarter of a wave and as long a chain),
+// up to rows of 2048 points; 4096 are 256 threads either way and 5 % faster at 16 points.
+// A step on 16 x 32 x 256 points: 104 us, 136-167 at 16 points a thread. Narrow and wide
+// on 64 x 64 x 64 (256 wide workgroups) 125 and 137 us, on 128 x 128 x 64 (1024) 253 and
+// 259, on 64 x 64 x 512 (2048) 384 and 351. At most 16 rows, which divide any grid's nx ny.
 constexpr int t_log2g(int log2l, bool wide) {
   const int g = (wide ? 10 : 8) - log2l;
   return g < 0 ? 0 : (g > 4 ? 4 : g);
 }
 
+constexpr int t_logr(int log2l, bool wide) { return wide || log2l > 11 ? 4 : 2; }
+
 template <int LOG2L>
 void dispatch_t_wide(bool wide, bool imaginary, int kind, long rows, hipStream_t s,
                      const TArgs& a, const cplx* tw) {
   constexpr int W = t_log2g(LOG2L, true), N = t_log2g(LOG2L, false);
+  using Wide = TStage<LOG2L, (1 << W), t_logr(LOG2L, true)>;
+  using Narrow = TStage<LOG2L, (1 << N), t_logr(LOG2L, false)>;
+  // A narrow workgroup fills a wave (but on rows of 4 and 8 points, 16 rows at most).
+  static_assert(RegsFft<LOG2L, (1 << N), false, false, t_logr(LOG2L, false)>::NT >=
+                (LOG2L < 4 ? 4 << LOG2L : 64));
   const unsigned blocks = static_cast<unsigned>(rows >> (wide ? W : N));
   if (wide && imaginary)
-    TStage<LOG2L, (1 << W)>::template launch<true>(kind, blocks, s, a, tw);
+    Wide::template launch<true>(kind, blocks, s, a, tw);
   else if (wide)
-    TStage<LOG2L, (1 << W)>::template launch<false>(kind, blocks, s, a, tw);
+    Wide::template launch<false>(kind, blocks, s, a, tw);
   else if (imaginary)
-    TStage<LOG2L, (1 << N)>::template launch<true>(kind, blocks, s, a, tw);
+    Narrow::template launch<true>(kind, blocks, s, a, tw);
   else
-    TStage<LOG2L, (1 << N)>::template launch<false>(kind, blocks, s, a, tw);
+    Narrow::template launch<false>(kind, blocks, s, a, tw);
 }
 
 void dispatch_t(int log2l, bool wide, bool imaginary, int kind, long rows, hipStream_t s,
@@ -349,12 +371,18 @@ int log2_of(int n) {
   return m;
 }
 
-// Sequences a workgroup of a strided pass owns: runs of up to 16 neighbouring points,
-// never more than `max_points` points in all.
-int axis_log2g(int n, long count, int max_points) {
+// Sequences (log2) a workgroup of a strided pass owns, of `count` neighbouring ones in each
+// of `blocks` blocks: runs of up to 16 points, never more than `max_points` points in all.
+// A short axis takes a wave of sequences where 256 workgroups remain: at 16 sequences of 8
+// points the y pass on 32 x 8 x 2048 ran workgroups of 8 threads and took 21 us, 7.4 in
+// LDS before. (16 points are 16 threads' butterflies and take what they took, 13.6 us on
+// 256 x 16 x 512.)
+int axis_log2g(int n, long count, long blocks, int max_points) {
   int g = 0;
-  const int cap = std::min(max_points, kMaxElems);
-  while (g < 4 && n * (1 << (g + 1)) <= cap && count % (1L << (g + 1)) == 0) ++g;
+  const int cap = std::min(max_points, kMaxElems), most = n <= kShortAxis ? 6 : 4;
+  while (g < most && n * (1 << (g + 1)) <= cap && count % (1L << (g + 1)) == 0 &&
+         (g < 4 || (count >> (g + 1)) * blocks >= 256))
+    ++g;
   return g;
 }
 
@@ -435,10 +463,10 @@ CartesianWorkspace::CartesianWorkspace(const sp_problem_desc& d) {
            "SOLPROP_MI355X_CARTESIAN_TILE is 4 to 4096 points");
   const long rows = static_cast<long>(nx_) * ny_;
   const int lt = log2_of(nt_);
-  wide_t_ = (rows >> t_log2g(lt, true)) >= 256;
+  wide_t_ = (rows >> t_log2g(lt, true)) >= 1024;
   t_blocks_ = static_cast<int>(rows >> t_log2g(lt, wide_t_));
-  gx_ = axis_log2g(nx_, nt_, max_points);
-  gy_ = axis_log2g(ny_, static_cast<long>(nx_) * nt_, max_points);
+  gx_ = axis_log2g(nx_, nt_, ny_, max_points);
+  gy_ = axis_log2g(ny_, static_cast<long>(nx_) * nt_, 1, max_points);
   try {
     SP_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     const int C = nx_ * ny_, N = nt_;

@@ -75,7 +75,7 @@ class CartesianWorkspace final : public Propagator {
   int gx_ = 0, gy_ = 0;  // log2 of the sequences a workgroup owns: x axis, y axis
   bool imaginary_ = false;  // the operator and prefactor tables have no real part
   const void *phi_ = nullptr, *pref_ = nullptr;
-  bool wide_t_ = true;   // the t rows' workgroups hold 2^11 points
+  bool wide_t_ = true;   // the t rows' workgroups hold 2^10 points, else 2^8
   int t_blocks_ = 0;
   std::size_t V_ = 0;
   DeviceProblem P_{};

@@ -15,7 +15,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("lossy", [False, True])
 @pytest.mark.parametrize("grid", [(4, 4, 4), (8, 4, 16), (4, 16, 2048), (512, 4, 8),
-                                  (16, 128, 64), (32, 32, 512), (128, 256, 8)])
+                                  (16, 128, 64), (32, 32, 512), (128, 256, 8),
+                                  # 64 and 32 sequences of 4 and 8 points, wide rows of 512
+                                  # points, narrow ones of 1024, rows of 4096
+                                  (64, 4, 256), (4, 256, 64), (8, 256, 32), (8, 64, 256),
+                                  (64, 32, 512), (16, 8, 1024), (4, 4, 4096)])
 def test_replay_at_the_edges_of_the_shapes(grid, lossy):
     print("Cartesian replay", grid, "lossy" if lossy else "lossless", flush=True)
     problem = problem_of(*grid)
