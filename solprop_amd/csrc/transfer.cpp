@@ -15,16 +15,26 @@ Transfer::~Transfer() {
   if (slots_) (void)hipHostFree(slots_);
 }
 
-bool Transfer::ready() {
-  if (slots_ || failed_) return !failed_;
+void Transfer::make_slots() {
   void* p = nullptr;
   bool ok = hipHostMalloc(&p, kLanes * kSlots * kChunk) == hipSuccess;
   for (auto& e : events_)
     ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-  slots_ = static_cast<char*>(p);
-  if (!ok) (void)hipGetLastError();
-  failed_ = !ok;
-  return ok;
+  if (ok) {
+    slots_ = static_cast<char*>(p);
+    return;
+  }
+  if (p) (void)hipHostFree(p);
+  (void)hipGetLastError();
+  failed_ = true;
+}
+
+// Whether a download of `bytes` goes through the slots, which it makes when they pay.
+bool Transfer::slots_for(std::size_t bytes) {
+  if (slots_ || failed_ || bytes < kDownload) return slots_ && bytes >= kDownload;
+  if (bytes >= kAtOnce || plain_ >= kRepaid) make_slots();
+  if (!slots_) plain_ += bytes;
+  return slots_ != nullptr;
 }
 
 // Runs lane(0) .. lane(kLanes - 1), each on a thread of its own where one can be had, and
@@ -58,9 +68,9 @@ void Transfer::run(F&& lane) {
 }
 
 void Transfer::upload(void* device, const void* host, std::size_t bytes, hipStream_t stream) {
-  if (bytes < kLeast || !ready()) {
-    SP_HIP(hipMemcpyAsync(device, host, bytes, hipMemcpyHostToDevice, stream));
+  if (bytes < kUpload || !slots_) {
     SP_HIP(hipStreamSynchronize(stream));
+    SP_HIP(hipMemcpy(device, host, bytes, hipMemcpyHostToDevice));
     return;
   }
   const std::size_t chunks = (bytes + kChunk - 1) / kChunk;
@@ -81,9 +91,9 @@ void Transfer::upload(void* device, const void* host, std::size_t bytes, hipStre
 }
 
 void Transfer::download(void* host, const void* device, std::size_t bytes, hipStream_t stream) {
-  if (bytes < kLeast || !ready()) {
-    SP_HIP(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, stream));
+  if (!slots_for(bytes)) {
     SP_HIP(hipStreamSynchronize(stream));
+    SP_HIP(hipMemcpy(host, device, bytes, hipMemcpyDeviceToHost));
     return;
   }
   const std::size_t chunks = (bytes + kChunk - 1) / kChunk;
