@@ -51,7 +51,6 @@ struct DeviceProblem {
   double plasma_cmr, plasma_ip;  // e^2/m_e and the ionisation potential, J
   double dt_fine, inv_T, inv_2T;
   const int* fine_to_coarse;   // (NF) coarse bin of each fine bin, -1 in the gaps
-  const int* crop;             // (N) fine bin of each coarse bin
   const unsigned char* active; // (N)
   const unsigned char* normmask;  // (N)
   const double* omega_window;  // (N)

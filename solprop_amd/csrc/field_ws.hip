@@ -163,9 +163,6 @@ void FieldWorkspace::allocate(const sp_problem_desc& d) {
   // The in-stage absorbers' stream (the temporal term, the transverse collar's product,
   // or their sum) follows the polarisation and, with plasma, the currents.
   P_.absorber_stream = absorbing() ? (d.has_plasma ? 3 : 1) : -1;
-  std::vector<int> crop(N);
-  for (int b = 0; b < N; ++b) crop[b] = b;
-  P_.crop = upload(crop.data(), crop.size());
   P_.active = upload(d.active_mask, N);
   P_.normmask = upload(d.norm_mask, N);
   P_.omega_window = upload(d.omega_window, N);

@@ -55,8 +55,13 @@ Workspace::Workspace(const sp_problem_desc& d) {
                d.projection && d.tableau_a && d.tableau_b && d.tableau_c && d.tableau_e,
            "a required problem array is missing");
   const int C = d.n_modes, N = d.n_omega, T = d.n_to;
-  for (int b = 0; b < N; ++b)
+  // The stage kernels visit the coarse bins from their fine ones, one each.
+  std::vector<int> f2c(T, -1);
+  for (int b = 0; b < N; ++b) {
     SP_CHECK(d.crop_index[b] >= 0 && d.crop_index[b] < T, "crop_index outside the fine grid");
+    SP_CHECK(f2c[d.crop_index[b]] < 0, "crop_index names a fine bin twice");
+    f2c[d.crop_index[b]] = b;
+  }
 
   for (int t = 0; t < d.n_phi; ++t) {
     phi_paths_.emplace_back();
@@ -129,13 +134,7 @@ Workspace::Workspace(const sp_problem_desc& d) {
   P_.inv_2T = 1.0 / (2.0 * T);
   P_.n_stages = d.n_stages;
 
-  std::vector<int> f2c(T, -1), crop(N);
-  for (int b = 0; b < N; ++b) {
-    crop[b] = static_cast<int>(d.crop_index[b]);
-    f2c[crop[b]] = b;
-  }
   P_.fine_to_coarse = device_copy(f2c.data(), f2c.size());
-  P_.crop = device_copy(crop.data(), crop.size());
   P_.active = device_copy(d.active_mask, N);
   P_.normmask = device_copy(d.norm_mask, N);
   P_.omega_window = device_copy(d.omega_window, N);

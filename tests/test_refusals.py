@@ -25,6 +25,15 @@ def test_envelope_under_adams_is_refused():
             "embedded Runge-Kutta")
 
 
+def test_envelope_bin_named_twice_is_refused():
+    p = gnlse_problem(n_t=64, window=1e-12)
+    crop = p.crop_index.copy()
+    crop[5] = crop[4]
+    refused(dataclasses.replace(p, crop_index=crop), "twice")
+    crop[5] = p.n_to
+    refused(dataclasses.replace(p, crop_index=crop), "outside the fine grid")
+
+
 def test_field_route_under_rk_is_refused():
     refused(dataclasses.replace(capillary_problem(n_t=256, n_nodes=4, integration="trapezoid"),
                                 method="rk"),
