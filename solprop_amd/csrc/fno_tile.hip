@@ -29,6 +29,15 @@ constexpr float kGeluC = 0.7978845608028654f;  // sqrt(2 / pi)
 constexpr float kGeluA = 0.044715f;
 constexpr int kRow = kTile + 8;  // an LDS row of a tile's bins (16-byte rows, banks spread)
 
+// LDS tiles are read 16 bytes a lane and written 8: the arrays start, and their rows lie,
+// on 16-byte lines.
+constexpr int kWide = 16;
+template <typename T>
+constexpr bool wide_pitch(int elements) {
+  return elements * sizeof(T) % kWide == 0;
+}
+static_assert(wide_pitch<bf16>(kRow));
+
 __device__ inline v8b load8(const bf16* p) { return *reinterpret_cast<const v8b*>(p); }
 
 __device__ inline bf16 bf(float x) {
@@ -113,8 +122,9 @@ template <int WP, int MP, bool LIFT, bool HEAD>
 __global__ void __launch_bounds__(256, 2) tile_layer(LayerArgs a) {
   constexpr int NC = WP / 32, KW = WP / 32, KM = MP / 32, MT = WP / 16, NT = MP / 64;
   constexpr int kCol = WP + 8;
-  __shared__ bf16 tile_cs[HEAD ? 1 : 2][HEAD ? 1 : WP * kRow];
-  __shared__ bf16 tile_sc[HEAD ? 2 : 1][HEAD ? kTile * kCol : 1];
+  static_assert(wide_pitch<bf16>(kCol));
+  __shared__ alignas(kWide) bf16 tile_cs[HEAD ? 1 : 2][HEAD ? 1 : WP * kRow];
+  __shared__ alignas(kWide) bf16 tile_sc[HEAD ? 2 : 1][HEAD ? kTile * kCol : 1];
   __shared__ float red[4];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
   const int ws = wave >> 1, wc = wave & 1;
@@ -319,7 +329,8 @@ struct MixArgs {
 template <int WP, int MP, bool BACK>
 __global__ void __launch_bounds__(256) tile_mix(MixArgs a) {
   constexpr int kCol = WP + 4;
-  __shared__ float in[2][16 * kCol];
+  __shared__ alignas(kWide) float in[2][16 * kCol];
+  static_assert(wide_pitch<float>(kCol));
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
   const int k = blockIdx.x, b0 = blockIdx.y * 16;
   const long plane = static_cast<long>(MP) * a.B * WP;
@@ -433,9 +444,10 @@ template <int WP>
 __global__ void __launch_bounds__(256, 1) tile_head_backward(HeadBackArgs a) {
   constexpr int NC = WP / 32, KW = WP / 32, MT = WP / 16;
   constexpr int kHid = kHeadUnits + 8;
-  __shared__ bf16 dh_hs[2][kHeadUnits * kRow];
-  __shared__ bf16 dh_sh[2][kTile * kHid];
-  __shared__ bf16 v_cs[2][WP * kRow];
+  static_assert(wide_pitch<bf16>(kHid));
+  __shared__ alignas(kWide) bf16 dh_hs[2][kHeadUnits * kRow];
+  __shared__ alignas(kWide) bf16 dh_sh[2][kTile * kHid];
+  __shared__ alignas(kWide) bf16 v_cs[2][WP * kRow];
   __shared__ float red[2 * kHeadUnits + WP + 1];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
   const int ws = wave >> 1, wc = wave & 1;
@@ -617,8 +629,8 @@ __global__ void __launch_bounds__(256, MODE == Back::kLayer ? 1 : 2)
   constexpr int NC = WP / 32, KW = WP / 32, KM = MP / 32, MT = WP / 16, NT = MP / 64;
   constexpr int kOwn = MT * MT / 4;  // tiles of the convolution's gradient a wave sums
   constexpr bool kTop = MODE == Back::kTop, kLift = MODE == Back::kLift;
-  __shared__ bf16 dz_cs[2][kLift ? 1 : WP * kRow];
-  __shared__ bf16 v_cs[2][kLift ? 1 : WP * kRow];
+  __shared__ alignas(kWide) bf16 dz_cs[2][kLift ? 1 : WP * kRow];
+  __shared__ alignas(kWide) bf16 v_cs[2][kLift ? 1 : WP * kRow];
   __shared__ float red[3 * WP];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
   const int ws = wave >> 1, wc = wave & 1;
