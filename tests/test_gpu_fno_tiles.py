@@ -2,8 +2,11 @@
 products of wider networks, against the FP64 oracle (``oracle/fno.py``).
 
 Channels pad to 32 or 64, twice the modes to 64 or 128, bins to tiles of 64 and samples
-to runs of 16; a batch splits each sample's tiles over workgroups by its size. The shapes
-below sit on and beside each of these edges. BF16 operands (unit roundoff 2^-9) pass
+to runs of 16. A batch splits each sample's tiles over some 512 workgroups forward and 256
+backward: small ones give a workgroup one tile, the larger ones below a run of two to
+eleven, whole or with a short last run, so that the buffers alternate and the spectral,
+weight and bias sums are kept over tiles (`test_runs_of_tiles` holds the splits). The shapes
+sit on and beside each of these edges. BF16 operands (unit roundoff 2^-9) pass
 through two products a layer forward and three back, so a tensor's relative error is a
 few 2^-9 sqrt(layers): the bounds are those of the other surrogate tests, 2 % and a cosine
 of 0.9995, which one wrong row, column or sign in a small tensor breaks.
@@ -30,7 +33,27 @@ EDGES = [
     (64, 65, 2, 128, 256, 4, 3),
     (65, 16, 2, 64, 256, 4, 3),
     (32, 16, 2, 129, 256, 4, 3),
+    # Runs of tiles: 4 and 8, 5 (2 at the end) and 11 (10), 3 (2, ragged bins) and 8, 3, 2.
+    (16, 8, 2, 32, 2048, 4, 64),
+    (48, 40, 2, 64, 2048, 4, 67),
+    (33, 33, 2, 127, 500, 4, 130),
+    (64, 64, 2, 128, 129, 4, 300),
+    (32, 32, 1, 16, 65, 1, 520),
 ]
+
+
+def tile_runs(n, batch, groups):
+    """Tiles a workgroup and in a sample's last one (``fno_tile.hip`` ``tile_split``)."""
+    tiles = -(-n // 64)
+    per = -(-tiles // max(1, min(tiles, groups // batch)))
+    return per, (tiles - 1) % per + 1
+
+
+def test_runs_of_tiles():
+    forward = {tile_runs(e[4], e[6], 512) for e in EDGES}
+    backward = {tile_runs(e[4], e[6], 256) for e in EDGES}
+    assert forward >= {(1, 1), (4, 4), (5, 2), (3, 2), (3, 3), (2, 2)}
+    assert backward >= {(1, 1), (8, 8), (11, 10), (3, 3), (2, 2)}
 
 
 @pytest.mark.parametrize("edge", EDGES, ids=lambda e: "-".join(map(str, e)))
