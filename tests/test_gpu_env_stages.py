@@ -85,6 +85,39 @@ def test_longest_sequences(n_t, ffac, option):
     assert abs(got - norm) <= norm_bound(problem, advanced, y0)
 
 
+# A weak launch without noise: the embedded pair's solutions agree to 1e-9 .. 1e-7 of the
+# tolerance, and their difference carries the rounding of the fields they are formed from.
+# The oracle's own norm moves by 1e-7 .. 1e-6 of itself when the launch moves by one unit in
+# the last place, so nothing closer can be asked of it: over six launches the device's root
+# mean square difference from the oracle is held to three times that movement (the same
+# arithmetic in another order rounds as much; six differences exceed thrice their standard
+# deviation in root mean square once in 1e8).
+@pytest.mark.parametrize("n_t", [512, 2048])
+@pytest.mark.parametrize("order", [1.0, 1.5])
+def test_weak_launch_norm_within_the_oracles_rounding(n_t, order):
+    print("envelope weak launch", n_t, order, flush=True)
+    problem = gnlse_problem(n_t=n_t, ffac=2, window=10e-12 * n_t / 8192, soliton_order=order,
+                            noise_model="none")
+    rng = np.random.default_rng(3)
+    dz = 1e-4
+    differences, movements = [], []
+    ws = Workspace(problem)
+    for _ in range(6):
+        launch = problem.field0 * (1.0 + rng.uniform(-0.05, 0.05))
+        problem_at = dataclasses.replace(problem, field0=launch)
+        _, norm, _ = oracle_trial(problem_at, dz)
+        differences.append(ws.probe(0.0, launch).trial(0.0, dz) - norm)
+        for _ in range(3):
+            moved = launch.copy()
+            parts = moved.view(np.float64)
+            parts *= 1.0 + np.finfo(np.float64).eps * rng.choice([-1, 0, 1], size=parts.shape)
+            movements.append(
+                oracle_trial(dataclasses.replace(problem, field0=moved), dz)[1] - norm)
+    ws.close()
+    assert 0.0 < norm < 1e-6
+    assert np.sqrt(np.mean(np.square(differences))) <= 3.0 * np.sqrt(np.mean(np.square(movements)))
+
+
 @pytest.mark.parametrize("option", ["raman", "absorber_noise", "varying_rate"])
 def test_commits_at_the_head_by_graph_and_direct(option, monkeypatch):
     problem = problem_of(1024, 2, option)
