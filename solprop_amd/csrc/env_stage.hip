@@ -24,7 +24,7 @@
 // What bounds a kernel is latency (its launch, one read of the input, the stages' LDS
 // hand-overs): 4 to 7 us each on 2^14 samples. An attempt of six stages with Raman on 2^13
 // bins and 2^14 samples took 322 us in 76 launches and takes 137 in 26; a trial of seven on
-// 2^16 bins and 2^17 samples took 845 and takes 460.
+// 2^16 bins and 2^17 samples took 845 and takes 427.
 #include "kernels.hpp"
 
 #include "fft_regs.hpp"

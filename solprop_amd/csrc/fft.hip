@@ -467,9 +467,13 @@ FftPlan::~FftPlan() {
 
 // One workgroup holds a whole row of up to kMaxElems points in one pass. For a few rows
 // that is a few CUs working through every stage in turn, and two passes over many CUs are
-// sooner done: a molecular trial's two source evaluations on 2^13 samples in three modes
-// 341 -> 334 us, 30 capillary attempts on 2^12 samples in four 2.66 -> 2.58 ms. From 18 rows
-// (six modes' streams) one pass is the shorter again (3.09 against 3.14 ms).
+// sooner done. An attempt of a capillary march in one pass and in two, on rows of 1024
+// points 68.3 and 67.6 us in one mode (1 row in, 3 out), 70.1 and 69.1 in four, 74.6 and
+// 70.9 in eight; of 2048 points 68.2 and 66.8, 70.4 and 67.8, 76.0 and 72.3; of 4096 points
+// 71.4 and 66.8, 74.1 and 68.8, 85.9 and 80.7. From 18 rows (six modes' streams) one pass is
+// the shorter again (30 attempts 3.09 against 3.14 ms). The instances of a scan share the
+// chip and would rather have one pass (96 of 2048-point rows in four modes: 905 us a round
+// against 955; of 4096, 1490 either way), but run their own marches' transforms, to the bit.
 constexpr std::size_t kFewRowsPoints = 1024, kFewRows = 16;
 
 void FftPlan::layout(std::size_t n, std::size_t batch, bool few_rows) {

@@ -624,8 +624,8 @@ struct BandLds {
 
 // The nodes a wave of the rate pass runs: on the modal route half as many as the other
 // band passes, for more waves to hide the loads' latency (at 2^14 samples and 128 nodes
-// 13.4 us, 15.6 with its nodes one after another); on the dense route (C = 0) as many
-// (26.8 us against 24.5 with two at the radial grid).
+// 13.3 us, 15.6 with its nodes one after another); on the dense route (C = 0) as many
+// (23.1 us against 23.8 with two at the radial grid).
 template <int C>
 constexpr int rate_nodes_per_wave() {
   return C == 0 ? kNodesPerWave : kNodesPerWave / 2;

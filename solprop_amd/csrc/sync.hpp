@@ -41,8 +41,9 @@ constexpr double kWaitLimitSeconds = 300.0;
 
 // Wait until `event` completes: spin for the first `spin_us` microseconds (a trial's
 // norms are wanted as soon as they land), then yield the core, then sleep for a 32nd of
-// the time waited so far, up to a millisecond: the event is seen at most 3 % late. (Steps
-// that doubled from 2 us overslept a 2.4 ms step by 0.9 ms.) A wait past kWaitLimitSeconds throws SP_BACKEND, so a
+// the time waited so far, up to a millisecond: the event is seen at most 3 % late, and by
+// what the host's timers add to a sleep (some 50 us). (Steps that doubled from 2 us
+// overslept a 2.4 ms step by 0.9 ms.) A wait past kWaitLimitSeconds throws SP_BACKEND, so a
 // device that never finishes cannot hold the host forever.
 inline void wait_event(hipEvent_t event, double spin_us = 200.0) {
   using clock = std::chrono::steady_clock;
