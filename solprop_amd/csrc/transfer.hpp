@@ -6,7 +6,7 @@
 // own, two each, so that the page faults, the host copies and the link overlap. State of
 // 8.4, 16.8, 33.6, 67 and 268 MB to the host, plain and in lanes: 0.49 and 0.36 ms, 1.02
 // and 0.62, 3.35 and 1.30, 6.8 and 2.4, 25.6 and 9.1. From pageable memory the plain copy
-// is as quick as the link but for the largest: 0.24 and 0.33, 0.46 and 0.60, 1.14 and 1.15,
+// is as quick as the link but for the largest: 0.24 and 0.33, 0.46 and 0.60, 1.15 and 1.14,
 // 2.26 and 2.20, 8.95 and 8.52 ms.
 //
 // The slots take 1.1 to 1.5 ms to make (a process's first pinned copy 5 ms more), so they
@@ -38,7 +38,7 @@ class Transfer {
   static constexpr int kSlots = 2;                   // a lane
   static constexpr std::size_t kChunk = 1UL << 20;   // bytes of a slot
   static constexpr std::size_t kDownload = 8UL << 20;  // the least that lanes are quicker for
-  static constexpr std::size_t kUpload = 64UL << 20;
+  static constexpr std::size_t kUpload = 32UL << 20;   // and the least to the device
   static constexpr std::size_t kAtOnce = 32UL << 20;   // a download that repays the slots
   static constexpr std::size_t kRepaid = 64UL << 20;   // plain downloads that would have
   bool slots_for(std::size_t bytes);

@@ -48,7 +48,7 @@ int main() {
     round_trip(t, s, 8 * MB + 1000, 99);
     fake::check(fake::copies - before == 1 + 9, "a plain upload and nine chunks back");
     // Every size through the slots: whole chunks, remainders, more than the lanes' slots.
-    for (std::size_t bytes : {8 * MB, 8 * MB + 16, 11 * MB - 48, 63 * MB, 64 * MB, 65 * MB + 80})
+    for (std::size_t bytes : {8 * MB, 8 * MB + 16, 11 * MB - 48, 31 * MB, 32 * MB, 33 * MB + 80})
       round_trip(t, s, bytes, static_cast<unsigned>(bytes));
     fake::check(fake::pinned_allocations == 1, "the slots are kept");
   }
