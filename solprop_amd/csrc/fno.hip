@@ -520,16 +520,24 @@ void transforms(const Shape& s, std::vector<bf16>& f, std::vector<bf16>& g) {
   f.resize(n * 2 * M);
   g.resize(2 * M * n);
   const double two_pi = 6.283185307179586;
+  std::vector<double> cosine(n), sine(n);  // the angles are n
+  for (long r = 0; r < n; ++r) {
+    const double a = two_pi * static_cast<double>(r) / static_cast<double>(n);
+    cosine[r] = std::cos(a);
+    sine[r] = std::sin(a);
+  }
   for (long t = 0; t < n; ++t)
-    for (long k = 0; k < M; ++k) {
-      const double a = two_pi * static_cast<double>((t * k) % n) / static_cast<double>(n);
-      const double c = std::cos(a), sn = std::sin(a);
-      const double w = (k == 0 ? 1.0 : 2.0) / static_cast<double>(n);
-      f[t * 2 * M + k] = to_bf16(static_cast<float>(c));
-      f[t * 2 * M + M + k] = to_bf16(static_cast<float>(-sn));
-      g[k * n + t] = to_bf16(static_cast<float>(w * c));
-      g[(M + k) * n + t] = to_bf16(static_cast<float>(-w * sn));
+    for (long k = 0, r = 0; k < M; ++k, r = (r + t) % n) {  // r = t k mod n
+      f[t * 2 * M + k] = to_bf16(static_cast<float>(cosine[r]));
+      f[t * 2 * M + M + k] = to_bf16(static_cast<float>(-sine[r]));
     }
+  for (long k = 0; k < M; ++k) {
+    const double w = (k == 0 ? 1.0 : 2.0) / static_cast<double>(n);
+    for (long t = 0, r = 0; t < n; ++t, r = (r + k) % n) {
+      g[k * n + t] = to_bf16(static_cast<float>(w * cosine[r]));
+      g[(M + k) * n + t] = to_bf16(static_cast<float>(-w * sine[r]));
+    }
+  }
 }
 
 }  // namespace
@@ -646,13 +654,14 @@ void Network::allocate_tiles() {
   // Both tables both ways round, the padded modes and bins zero.
   std::vector<bf16> table[4];  // g_s, f_k, f_s, g_k
   for (auto& v : table) v.assign(NP * MP, 0);
-  for (long k = 0; k < 2 * M; ++k) {
-    const long kp = k < M ? k : MP / 2 + k - M;
-    for (long x = 0; x < n; ++x) {
-      table[0][x * MP + kp] = table[3][kp * NP + x] = g[k * n + x];
-      table[1][kp * NP + x] = table[2][x * MP + kp] = f[x * 2 * M + k];
+  for (long x0 = 0; x0 < n; x0 += 64)  // by blocks of bins: one side of each pair is strided
+    for (long k = 0; k < 2 * M; ++k) {
+      const long kp = k < M ? k : MP / 2 + k - M;
+      for (long x = x0; x < std::min(n, x0 + 64); ++x) {
+        table[0][x * MP + kp] = table[3][kp * NP + x] = g[k * n + x];
+        table[1][kp * NP + x] = table[2][x * MP + kp] = f[x * 2 * M + k];
+      }
     }
-  }
   bf16** to[4] = {&b.g_s, &b.f_k, &b.f_s, &b.g_k};
   for (int i = 0; i < 4; ++i) {
     *to[i] = alloc<bf16>(NP * MP);
